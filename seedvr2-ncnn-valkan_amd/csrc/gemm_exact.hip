@@ -11,15 +11,17 @@
 // the reference tree): against it this product is pinned by the closed form
 // y = W x + b only, not bit for bit.
 //
-// On the VALU in fp64 (an fp64 MFMA would sum four products per step in its
-// own order).  Two forms of the same arithmetic:
-//   * tiled (rows > 16): one 256-thread workgroup per 64 x 128 tile of y;
-//     each thread keeps an 8 x 4 block of double accumulators; k moves
-//     through LDS in stages of 8, held as double, two stages in flight;
+// Two forms of the same arithmetic:
+//   * tiled (rows > 16): v_mfma_f64_16x16x4_f64.  The instruction adds its
+//     four products to an accumulator one after another in increasing k, each
+//     a fused multiply-add with its own rounding (tests/test_gpu_exact.py
+//     pins the product bit for bit), so it is the same sum as a chain of
+//     scalar ones.  A lane supplies two doubles for 16 multiply-adds where
+//     the VALU form, an 8 x 4 block a thread, read 12 doubles of LDS for 32:
+//     LDS reads bounded that one at 25 TFLOP/s;
 //   * few rows (rows <= 16, e.g. the DiT's one-row time MLP): one one-wave
-//     workgroup per 16 output columns, so a wide product spreads over many
-//     CUs and several workgroups share each; W moves through LDS in chunks of
-//     64 k, transposed, the next chunk loaded into registers meanwhile.
+//     workgroup per 16 output columns and one such MFMA tile, so a wide
+//     product spreads over many CUs; chunks of 64 k, four of them in flight.
 #include "sv2_internal.h"
 
 namespace sv2
@@ -27,188 +29,258 @@ namespace sv2
 namespace
 {
 
-constexpr int kBM = 64;   // rows of y per workgroup
-constexpr int kBN = 128;  // output columns per workgroup
-constexpr int kBK = 8;    // k per LDS stage
-constexpr int kTM = 8;    // rows per thread
-constexpr int kTN = 4;    // columns per thread
+typedef __attribute__((ext_vector_type(4))) double d4;
 
+constexpr int kBN = 64;        // output columns per workgroup
+constexpr int kBK = 32;        // k per LDS stage
+constexpr int kStride = 36;    // floats per staged row: 32 + 4, 16 consecutive rows on distinct banks
+constexpr int kFill = 1024;    // workgroups of 64 rows from which 64-row tiles are taken
+
+// One workgroup of four waves per BM x 64 tile of y, wave (r, c) = (wave / 2,
+// wave % 2) a (BM / 2) x 32 block.  A stage of 32 k is held in LDS as fp32 in
+// the order an MFMA lane consumes it: lane group q = lane / 16 multiplies k =
+// 4 s + q at step s, so k sits at position 8 (k % 4) + k / 4 of its row and a
+// lane's eight steps are two 16-byte reads.  The next stage is loaded into
+// registers while the current one is multiplied.
+//
+// Bound by the fp64 matrix rate (45 to 47 TFLOP/s measured with nothing but
+// this instruction, two waves or more per SIMD; one wave per SIMD gives 34,
+// hence the small tiles).
+template <int BM>
 __global__ __launch_bounds__(256) void gemm_f32_exact_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                              const float* __restrict__ bias, float* __restrict__ y,
                                                              int rows, int in, int out)
 {
-    __shared__ double xs[2][kBK][kBM];
-    __shared__ double ws[2][kBK][kBN];
+    constexpr int kMT = BM / 32;       // 16-row tiles per wave
+    constexpr int kXQ = BM * kBK / 4 / 256; // float4 of x per thread and stage
+    constexpr int kWQ = kBN * kBK / 4 / 256;
+    __shared__ __attribute__((aligned(16))) float xs[2][BM * kStride];
+    __shared__ __attribute__((aligned(16))) float ws[2][kBN * kStride];
     const int tid = threadIdx.x;
-    const int tx = tid & 31; // columns 4 tx .. 4 tx + 3
-    const int ty = tid >> 5; // rows 8 ty .. 8 ty + 7
-    const int row0 = blockIdx.y * kBM;
-    const int col0 = blockIdx.x * kBN;
+    const int lane = tid & 63;
+    const int wave = tid >> 6;
+    const int lr = lane & 15;
+    const int lq = lane >> 4;
+    // the row bands of one column tile run side by side and share its W rows
+    const long long id = static_cast<long long>(blockIdx.y) * gridDim.x + blockIdx.x;
+    const long long row0 = id % gridDim.y * BM;
+    const long long col0 = id / gridDim.y * kBN;
+    const bool quads = (in & 3) == 0 && ((reinterpret_cast<size_t>(x) | reinterpret_cast<size_t>(w)) & 15) == 0;
 
-    // staging assignment: x tile 64 rows x 8 k (2 per thread), w tile 128
-    // columns x 8 k (4 per thread); values past the edges are zero (their
-    // products are +0 and leave the sums unchanged)
-    const int xr = tid >> 2;
-    const int xk = (tid & 3) * 2;
-    const int wc = tid >> 1;
-    const int wk = (tid & 1) * 4;
-    const bool x_row_ok = row0 + xr < rows;
-    const bool w_col_ok = col0 + wc < out;
-    const float* xp = x + static_cast<long long>(x_row_ok ? row0 + xr : 0) * in;
-    const float* wp = w + static_cast<long long>(w_col_ok ? col0 + wc : 0) * in;
-
-    auto stage = [&](int buf, int k0) {
-#pragma unroll
-        for (int e = 0; e < 2; e++)
+    // thread: k 4 (tid % 8) .. + 3 of rows tid / 8 + 32 i.  Values past the
+    // edges are zero (their products are +0 and leave the sums unchanged)
+    const int kq = tid & 7;
+    const int sr = tid >> 3;
+    float4 xv[kXQ], wv[kWQ];
+    auto load1 = [&](const float* base, long long row, long long limit, int k) {
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (row < limit && k < in)
         {
-            const int k = k0 + xk + e;
-            xs[buf][xk + e][xr] = (x_row_ok && k < in) ? static_cast<double>(xp[k]) : 0.0;
+            const float* p = base + row * in + k;
+            if (quads)
+                return *reinterpret_cast<const float4*>(p);
+            v.x = p[0];
+            v.y = k + 1 < in ? p[1] : 0.f;
+            v.z = k + 2 < in ? p[2] : 0.f;
+            v.w = k + 3 < in ? p[3] : 0.f;
         }
+        return v;
+    };
+    auto load = [&](int k0) {
 #pragma unroll
-        for (int e = 0; e < 4; e++)
-        {
-            const int k = k0 + wk + e;
-            ws[buf][wk + e][wc] = (w_col_ok && k < in) ? static_cast<double>(wp[k]) : 0.0;
-        }
+        for (int i = 0; i < kXQ; i++)
+            xv[i] = load1(x, row0 + sr + 32 * i, rows, k0 + 4 * kq);
+#pragma unroll
+        for (int i = 0; i < kWQ; i++)
+            wv[i] = load1(w, col0 + sr + 32 * i, out, k0 + 4 * kq);
+    };
+    auto put = [&](float* dst, const float4& v) {
+        dst[0] = v.x;
+        dst[8] = v.y;
+        dst[16] = v.z;
+        dst[24] = v.w;
+    };
+    auto store = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < kXQ; i++)
+            put(&xs[buf][(sr + 32 * i) * kStride + kq], xv[i]);
+#pragma unroll
+        for (int i = 0; i < kWQ; i++)
+            put(&ws[buf][(sr + 32 * i) * kStride + kq], wv[i]);
     };
 
-    double acc[kTM][kTN];
+    const int wr = (wave >> 1) * (BM / 2);
+    const int wc = (wave & 1) * 32;
+    d4 acc[kMT][2];
 #pragma unroll
-    for (int i = 0; i < kTM; i++)
+    for (int i = 0; i < kMT; i++)
 #pragma unroll
-        for (int j = 0; j < kTN; j++)
-            acc[i][j] = 0.0;
+        for (int j = 0; j < 2; j++)
+            acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
 
     const int nk = (in + kBK - 1) / kBK;
-    stage(0, 0);
+    load(0);
+    store(0);
     __syncthreads();
     for (int s = 0; s < nk; s++)
     {
         const int buf = s & 1;
         if (s + 1 < nk)
-            stage(buf ^ 1, (s + 1) * kBK);
+            load((s + 1) * kBK);
 #pragma unroll
-        for (int k = 0; k < kBK; k++)
+        for (int h = 0; h < 2; h++)
         {
-            double a[kTM];
-            double b[kTN];
+            float4 a[kMT], b[2];
 #pragma unroll
-            for (int i = 0; i < kTM; i++)
-                a[i] = xs[buf][k][ty * kTM + i];
+            for (int i = 0; i < kMT; i++)
+                a[i] = *reinterpret_cast<const float4*>(&xs[buf][(wr + 16 * i + lr) * kStride + 8 * lq + 4 * h]);
 #pragma unroll
-            for (int j = 0; j < kTN; j++)
-                b[j] = ws[buf][k][tx * kTN + j];
+            for (int j = 0; j < 2; j++)
+                b[j] = *reinterpret_cast<const float4*>(&ws[buf][(wc + 16 * j + lr) * kStride + 8 * lq + 4 * h]);
 #pragma unroll
-            for (int i = 0; i < kTM; i++)
+            for (int e = 0; e < 4; e++)
 #pragma unroll
-                for (int j = 0; j < kTN; j++)
-                    acc[i][j] = __builtin_fma(a[i], b[j], acc[i][j]);
+                for (int i = 0; i < kMT; i++)
+#pragma unroll
+                    for (int j = 0; j < 2; j++)
+                        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                            static_cast<double>((&a[i].x)[e]), static_cast<double>((&b[j].x)[e]), acc[i][j], 0, 0, 0);
         }
+        // the other buffer's readers passed the last barrier
+        if (s + 1 < nk)
+            store(buf ^ 1);
         __syncthreads();
     }
 
-    double bv[kTN];
+    // register e of a tile: row 4 e + lane / 16, column lane % 16
 #pragma unroll
-    for (int j = 0; j < kTN; j++)
+    for (int j = 0; j < 2; j++)
     {
-        const int c = col0 + tx * kTN + j;
-        bv[j] = (bias && c < out) ? static_cast<double>(bias[c]) : 0.0;
-    }
+        const long long c = col0 + wc + 16 * j + lr;
+        if (c >= out)
+            continue;
+        const double bv = bias ? static_cast<double>(bias[c]) : 0.0;
 #pragma unroll
-    for (int i = 0; i < kTM; i++)
-    {
-        const int r = row0 + ty * kTM + i;
-        if (r >= rows)
-            break;
-        float* yr = y + static_cast<long long>(r) * out;
+        for (int i = 0; i < kMT; i++)
 #pragma unroll
-        for (int j = 0; j < kTN; j++)
-        {
-            const int c = col0 + tx * kTN + j;
-            if (c < out)
-                yr[c] = static_cast<float>(acc[i][j] + bv[j]);
-        }
+            for (int e = 0; e < 4; e++)
+            {
+                const long long r = row0 + wr + 16 * i + 4 * e + lq;
+                if (r < rows)
+                    y[r * out + c] = static_cast<float>(acc[i][j][e] + bv);
+            }
     }
 }
 
 constexpr int kRowsSmall = 16; // the few-rows form handles up to this many rows
 constexpr int kCols = 16;      // output columns per few-rows workgroup (one wave)
-constexpr int kChunk = 64;     // k per LDS chunk of the few-rows form
+constexpr int kChunk = 64;     // k per chunk of the few-rows form
+constexpr int kAhead = 4;      // chunks in flight
+constexpr int kChunkStride = kChunk + 4;
 
-// One wave: lane (c, s) = (lane % 16, lane / 16) owns column col0 + c for
-// rows s, s + 4, s + 8, s + 12.  Lane l stages 16 consecutive k of W row
-// col0 + l / 4, and loads the next chunk's into registers while the current
-// chunk is summed; several of these small workgroups share a CU and hide
-// each other's loads.
+// One wave: one 16 x 16 MFMA tile, rows of x by 16 output columns.  Lane l
+// loads k 16 (l % 4) .. + 15 of row l / 4 of a chunk, four chunks ahead, into
+// registers; a chunk goes through the wave's LDS into the lane order of the
+// MFMA (k at position 16 (k % 4) + k / 4 of its row).  A workgroup is one
+// wave, whose LDS operations complete in order: no barrier.
+//
+// An output's 2560 sums are one chain of 640 dependent MFMAs, which bounds the
+// DiT's square time product (2560 -> 2560, one row); the wide one (2560 ->
+// 15360) is the stream of its 157 MB of weights.
 __global__ __launch_bounds__(64) void gemv_f32_exact_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                             const float* __restrict__ bias, float* __restrict__ y,
                                                             int rows, int in, int out)
 {
-    __shared__ float wt[kChunk][kCols];      // wt[k][c] = W[col0 + c][k0 + k]
-    __shared__ float xs[kRowsSmall][kChunk]; // xs[r][k] = x[r][k0 + k]
+    __shared__ __attribute__((aligned(16))) float wt[kCols * kChunkStride];
+    __shared__ __attribute__((aligned(16))) float xt[kRowsSmall * kChunkStride];
     const int lane = threadIdx.x;
-    const int c = lane & (kCols - 1);
-    const int slot = lane >> 4;
+    const int lr = lane & 15;
+    const int lq = lane >> 4;
     const int col0 = blockIdx.x * kCols;
-    const int wr = lane >> 2;
-    const int wk = (lane & 3) * 16;
-    const bool w_ok = col0 + wr < out;
-    const float* wp = w + static_cast<long long>(w_ok ? col0 + wr : 0) * in;
+    const int sr = lane >> 2;
+    const int sk = (lane & 3) * 16;
+    const bool w_ok = col0 + sr < out;
+    const bool x_ok = sr < rows;
+    const float* wp = w + static_cast<long long>(w_ok ? col0 + sr : 0) * in;
+    const float* xp = x + static_cast<long long>(x_ok ? sr : 0) * in;
+    const bool quads = (in & 3) == 0 && ((reinterpret_cast<size_t>(x) | reinterpret_cast<size_t>(w)) & 15) == 0;
 
     // values past the edges are zero: their products are +0 and the running
     // sums, which start at +0, stay what they were
-    float wv[16];
-    auto load_w = [&](int k0) {
+    auto load = [&](const float* p, bool ok, int k0, float4 (&v)[4]) {
 #pragma unroll
-        for (int e = 0; e < 16; e++)
+        for (int e = 0; e < 4; e++)
         {
-            const int k = k0 + wk + e;
-            wv[e] = (w_ok && k < in) ? wp[k] : 0.f;
+            const int k = k0 + sk + 4 * e;
+            v[e] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (!ok || k >= in)
+                continue;
+            if (quads)
+            {
+                v[e] = *reinterpret_cast<const float4*>(p + k);
+                continue;
+            }
+            v[e].x = p[k];
+            v[e].y = k + 1 < in ? p[k + 1] : 0.f;
+            v[e].z = k + 2 < in ? p[k + 2] : 0.f;
+            v[e].w = k + 3 < in ? p[k + 3] : 0.f;
+        }
+    };
+    auto put = [&](float* dst, const float4 (&v)[4]) {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+        {
+            float* d = dst + (sk >> 2) + e;
+            d[0] = v[e].x;
+            d[16] = v[e].y;
+            d[32] = v[e].z;
+            d[48] = v[e].w;
         }
     };
 
-    double acc[kRowsSmall / 4];
+    d4 acc = {0.0, 0.0, 0.0, 0.0};
+    float4 wv[kAhead][4], xv[kAhead][4];
 #pragma unroll
-    for (int i = 0; i < kRowsSmall / 4; i++)
-        acc[i] = 0.0;
-
-    load_w(0);
-    for (int k0 = 0; k0 < in; k0 += kChunk)
+    for (int a = 0; a < kAhead; a++)
     {
-#pragma unroll
-        for (int e = 0; e < 16; e++)
-            wt[wk + e][wr] = wv[e];
-#pragma unroll
-        for (int j = 0; j < kRowsSmall * kChunk / 64; j++)
-        {
-            const int i = lane + 64 * j;
-            const int r = i / kChunk;
-            const int k = k0 + i % kChunk;
-            xs[r][i % kChunk] = (r < rows && k < in) ? x[static_cast<long long>(r) * in + k] : 0.f;
-        }
-        __syncthreads();
-        if (k0 + kChunk < in)
-            load_w(k0 + kChunk);
-#pragma unroll
-        for (int i = 0; i < kRowsSmall / 4; i++)
-        {
-            if (slot + 4 * i >= rows) // rows past the input: nothing to sum
-                break;
-#pragma unroll 16
-            for (int k = 0; k < kChunk; k++)
-                acc[i] = __builtin_fma(static_cast<double>(xs[slot + 4 * i][k]), static_cast<double>(wt[k][c]), acc[i]);
-        }
-        __syncthreads();
+        load(wp, w_ok, a * kChunk, wv[a]);
+        load(xp, x_ok, a * kChunk, xv[a]);
     }
-    if (col0 + c >= out)
-        return;
-    const double bv = bias ? static_cast<double>(bias[col0 + c]) : 0.0;
-#pragma unroll
-    for (int i = 0; i < kRowsSmall / 4; i++)
+    for (int k0 = 0; k0 < in; k0 += kAhead * kChunk)
     {
-        const int r = slot + 4 * i;
+#pragma unroll
+        for (int a = 0; a < kAhead; a++)
+        {
+            // chunks past the last are zero: their products change nothing
+            put(&wt[sr * kChunkStride], wv[a]);
+            put(&xt[sr * kChunkStride], xv[a]);
+            __builtin_amdgcn_wave_barrier();
+            load(wp, w_ok, k0 + (a + kAhead) * kChunk, wv[a]);
+            load(xp, x_ok, k0 + (a + kAhead) * kChunk, xv[a]);
+            float4 wf[4], xf[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+            {
+                wf[e] = *reinterpret_cast<const float4*>(&wt[lr * kChunkStride + 16 * lq + 4 * e]);
+                xf[e] = *reinterpret_cast<const float4*>(&xt[lr * kChunkStride + 16 * lq + 4 * e]);
+            }
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int s = 0; s < 16; s++)
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(static_cast<double>((&xf[s >> 2].x)[s & 3]),
+                                                           static_cast<double>((&wf[s >> 2].x)[s & 3]), acc, 0, 0, 0);
+        }
+    }
+    const int c = col0 + lr;
+    if (c >= out)
+        return;
+    const double bv = bias ? static_cast<double>(bias[c]) : 0.0;
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+    {
+        const int r = 4 * e + lq;
         if (r < rows)
-            y[static_cast<long long>(r) * out + col0 + c] = static_cast<float>(acc[i] + bv);
+            y[static_cast<long long>(r) * out + c] = static_cast<float>(acc[e] + bv);
     }
 }
 
@@ -230,10 +302,17 @@ int gemm_f32_exact(hipStream_t stream, int rows, int in, int out, const float* x
         const hipError_t err = hipGetLastError();
         return err == hipSuccess ? SV2_OK : hip_error(err, "gemv_f32_exact_kernel launch");
     }
-    const dim3 grid(static_cast<unsigned>((out + kBN - 1) / kBN), static_cast<unsigned>((rows + kBM - 1) / kBM));
-    if (grid.y > 65535u)
+    const unsigned bands = (static_cast<unsigned>(rows) + 63u) / 64u;
+    const unsigned cols = (static_cast<unsigned>(out) + kBN - 1) / kBN;
+    if (bands > 65535u)
         return set_error(SV2_EUNSUPPORTED, "inner product (fp32): too many rows");
-    hipLaunchKernelGGL(gemm_f32_exact_kernel, grid, dim3(256), 0, stream, x, w, bias, y, rows, in, out);
+    // 32-row tiles where 64-row ones would give few workgroups per CU
+    if (static_cast<long long>(bands) * cols >= kFill)
+        hipLaunchKernelGGL(gemm_f32_exact_kernel<64>, dim3(cols, bands), dim3(256), 0, stream, x, w, bias, y, rows,
+                           in, out);
+    else
+        hipLaunchKernelGGL(gemm_f32_exact_kernel<32>, dim3(cols, (static_cast<unsigned>(rows) + 31u) / 32u), dim3(256),
+                           0, stream, x, w, bias, y, rows, in, out);
     const hipError_t err = hipGetLastError();
     return err == hipSuccess ? SV2_OK : hip_error(err, "gemm_f32_exact_kernel launch");
 }

@@ -60,6 +60,19 @@ def test_inner_product_f32_bit_exact(hip, orc, device, rows, k, n, bias):
     assert nd <= 2
 
 
+@pytest.mark.parametrize("rows,k,n,bias", [
+    (2, 1, 17, True),          # one product, one column past a tile
+    (16, 257, 33, False),      # few rows: one k past four chunks, rows not 16-byte aligned
+    (5, 64, 16, True),         # few rows: one chunk of the four in flight
+    (31, 31, 63, True),        # 32-row tiles, one short of every edge
+    (33, 33, 65, False),       # 32-row tiles, one past every edge
+    (1030, 36, 4130, True),    # 64-row tiles, ragged on both sides
+    (4033, 32, 1024, False),   # 64-row tiles, one stage
+])
+def test_inner_product_f32_tile_edges(hip, orc, device, rows, k, n, bias):
+    test_inner_product_f32_bit_exact(hip, orc, device, rows, k, n, bias)
+
+
 def exact_case(hip, orc, device, *, T, H, W, Lt, heads, shifted=False, wt=0, wh=0, ww=0, qk_norm=True,
                rope_mode=0, out_dtype="f32", seed=0, video_windows=None):
     print(f"[exact attention] T={T} H={H} W={W} Lt={Lt} heads={heads} shifted={shifted} win=({wt},{wh},{ww}) "
