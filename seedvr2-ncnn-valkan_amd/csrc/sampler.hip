@@ -21,6 +21,7 @@ namespace
 
 constexpr int kThreads = 256;
 constexpr int kReduceBlocks = 1024; // partial sums of the guidance statistics
+constexpr int kScaleBlocks = 256;   // blocks of the rescale, one per CU
 
 unsigned blocks_for(long long n)
 {
@@ -46,56 +47,91 @@ __global__ __launch_bounds__(kThreads) void condition_kernel(const float* a, con
     out[i] = left + right;
 }
 
+// Four consecutive fp32 elements of an array of any float alignment.
+typedef __attribute__((ext_vector_type(4), aligned(4))) float f4;
+
+// A thread takes four consecutive elements: the arrays stream in 16-byte
+// accesses, and a launch's blocks fall to a quarter.
+unsigned blocks_for_quads(long long n)
+{
+    return blocks_for((n + 3) / 4);
+}
+
 // engine.cpp:125-149: channels 0-15 the latent, 16-31 the condition, 32 ones.
-// Channel-major: [16][tokens] sources into [33][tokens] (the CPU engine);
-// token-major: [tokens][16] sources into [tokens][33] (sampler.cpp:337-357).
+// Channel-major ([16][tokens] sources into [33][tokens], the CPU engine): the
+// output is the latent, the condition and a channel of ones one after the
+// other, copied in quads (no channel index: with one 64-bit division an
+// element the 720p clip's input took 7.5 us).
 __global__ __launch_bounds__(kThreads) void dit_input_kernel(const float* latent, const float* condition, float* out,
-                                                             long long tokens, int channel_major)
+                                                             long long tokens)
+{
+    const long long i = 4 * (static_cast<long long>(blockIdx.x) * kThreads + threadIdx.x);
+    const long long n = 16 * tokens; // a multiple of four: no quad crosses a source
+    if (i < 2 * n)
+    {
+        const float* src = i < n ? latent + i : condition + (i - n);
+        *reinterpret_cast<f4*>(out + i) = *reinterpret_cast<const f4*>(src);
+        return;
+    }
+    for (long long k = i; k < min(i + 4, 33 * tokens); k++)
+        out[k] = 1.0f;
+}
+
+// Token-major: [tokens][16] sources into [tokens][33] (sampler.cpp:337-357).
+__global__ __launch_bounds__(kThreads) void dit_input_tokens_kernel(const float* latent, const float* condition,
+                                                                    float* out, long long tokens)
 {
     const long long i = static_cast<long long>(blockIdx.x) * kThreads + threadIdx.x;
     if (i >= 33 * tokens)
         return;
-    long long c, t;
-    if (channel_major)
-    {
-        c = i / tokens;
-        t = i - c * tokens;
-        out[i] = c < 16 ? latent[c * tokens + t] : (c < 32 ? condition[(c - 16) * tokens + t] : 1.0f);
-    }
-    else
-    {
-        t = i / 33;
-        c = i - t * 33;
-        out[i] = c < 16 ? latent[t * 16 + c] : (c < 32 ? condition[t * 16 + c - 16] : 1.0f);
-    }
+    const long long t = i / 33;
+    const long long c = i - t * 33;
+    out[i] = c < 16 ? latent[t * 16 + c] : (c < 32 ? condition[t * 16 + c - 16] : 1.0f);
 }
 
-// sampler.cpp:217-218: neg + scale * (pos - neg); with `partial` (the
-// rescale), each block also writes its double sums of pos, pos^2, out, out^2
-// (grid-stride over the elements, fixed order per block).
+// sampler.cpp:217-218: neg + scale * (pos - neg)
+__device__ inline float guide(float p, float n, float scale)
+{
+    const float diff = p - n;
+    const float scaled = scale * diff;
+    return n + scaled;
+}
+
 __global__ __launch_bounds__(kThreads) void cfg_kernel(const float* pos, const float* neg, float* out,
-                                                       long long count, float scale, double* partial)
+                                                       long long count, float scale)
+{
+    const long long i = 4 * (static_cast<long long>(blockIdx.x) * kThreads + threadIdx.x);
+    if (i + 4 <= count)
+    {
+        const f4 p = *reinterpret_cast<const f4*>(pos + i);
+        const f4 n = *reinterpret_cast<const f4*>(neg + i);
+        f4 o;
+        for (int e = 0; e < 4; e++)
+            o[e] = guide(p[e], n[e], scale);
+        *reinterpret_cast<f4*>(out + i) = o;
+        return;
+    }
+    for (long long k = i; k < count; k++)
+        out[k] = guide(pos[k], neg[k], scale);
+}
+
+// With the rescale each block also writes its double sums of pos, pos^2, out,
+// out^2 (grid-stride over the elements, fixed order per block).
+__global__ __launch_bounds__(kThreads) void cfg_sums_kernel(const float* pos, const float* neg, float* out,
+                                                            long long count, float scale, double* partial)
 {
     double sp = 0.0, spp = 0.0, so = 0.0, soo = 0.0;
     const long long stride = static_cast<long long>(gridDim.x) * kThreads;
     for (long long i = static_cast<long long>(blockIdx.x) * kThreads + threadIdx.x; i < count; i += stride)
     {
         const float p = pos[i];
-        const float n = neg[i];
-        const float diff = p - n;
-        const float scaled = scale * diff;
-        const float o = n + scaled;
+        const float o = guide(p, neg[i], scale);
         out[i] = o;
-        if (partial)
-        {
-            sp += p;
-            spp += static_cast<double>(p) * p;
-            so += o;
-            soo += static_cast<double>(o) * o;
-        }
+        sp += p;
+        spp += static_cast<double>(p) * p;
+        so += o;
+        soo += static_cast<double>(o) * o;
     }
-    if (!partial)
-        return;
     __shared__ double red[4][kThreads];
     red[0][threadIdx.x] = sp;
     red[1][threadIdx.x] = spp;
@@ -114,14 +150,18 @@ __global__ __launch_bounds__(kThreads) void cfg_kernel(const float* pos, const f
 }
 
 // sampler.cpp:41-62 (unbiased standard deviation from the sums) and :219-235:
-// factor = rescale * std(pos) / std(out) + (1 - rescale) when std(out) > 0.
-// One block: thread t adds the partials of blocks t, t + 256, ... in that
-// order, then a fixed tree over the threads, so the factor does not depend
-// on scheduling.  factor_out[0] = factor, [1] = 1 when it applies.
-__global__ __launch_bounds__(kThreads) void cfg_factor_kernel(const double* partial, int nblocks, long long count,
-                                                              float rescale, float* factor_out)
+// factor = rescale * std(pos) / std(out) + (1 - rescale) when std(out) > 0,
+// then the outputs times it.  Every block forms the factor itself (a launch
+// of one block for it cost 2.8 us of the small clip's 13): thread t adds the
+// partials of blocks t, t + 256, ... in that order, then a fixed tree over the
+// threads, so the factor is the same in all of them and does not depend on
+// scheduling.  At most kScaleBlocks blocks, each reading the partials (32 KB
+// at most) once.
+__global__ __launch_bounds__(kThreads) void cfg_scale_kernel(const double* partial, int nblocks, float* out,
+                                                             long long count, float rescale)
 {
     __shared__ double red[4][kThreads];
+    __shared__ float factor[2];
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
     for (int b = threadIdx.x; b < nblocks; b += kThreads)
         for (int k = 0; k < 4; k++)
@@ -136,58 +176,75 @@ __global__ __launch_bounds__(kThreads) void cfg_factor_kernel(const double* part
                 red[k][threadIdx.x] += red[k][threadIdx.x + s];
         __syncthreads();
     }
-    if (threadIdx.x != 0)
-        return;
-    const double sp = red[0][0], spp = red[1][0], so = red[2][0], soo = red[3][0];
-    double std_pos = 0.0, std_out = 0.0;
-    if (count > 1)
+    if (threadIdx.x == 0)
     {
-        const double n = static_cast<double>(count);
-        std_pos = sqrt(fmax(0.0, (spp - sp * sp / n) / (n - 1)));
-        std_out = sqrt(fmax(0.0, (soo - so * so / n) / (n - 1)));
-    }
-    if (std_out > 0.0)
-    {
-        factor_out[0] = static_cast<float>(static_cast<double>(rescale) * std_pos / std_out +
+        const double sp = red[0][0], spp = red[1][0], so = red[2][0], soo = red[3][0];
+        double std_pos = 0.0, std_out = 0.0;
+        if (count > 1)
+        {
+            const double n = static_cast<double>(count);
+            std_pos = sqrt(fmax(0.0, (spp - sp * sp / n) / (n - 1)));
+            std_out = sqrt(fmax(0.0, (soo - so * so / n) / (n - 1)));
+        }
+        factor[0] = 1.0f;
+        factor[1] = 0.0f;
+        if (std_out > 0.0)
+        {
+            factor[0] = static_cast<float>(static_cast<double>(rescale) * std_pos / std_out +
                                            static_cast<double>(1.0f - rescale));
-        factor_out[1] = 1.0f;
+            factor[1] = 1.0f;
+        }
     }
-    else
-    {
-        factor_out[0] = 1.0f;
-        factor_out[1] = 0.0f;
-    }
-}
-
-__global__ __launch_bounds__(kThreads) void cfg_scale_kernel(float* out, long long count, const float* factor)
-{
-    const long long i = static_cast<long long>(blockIdx.x) * kThreads + threadIdx.x;
-    if (i >= count || factor[1] == 0.0f)
+    __syncthreads();
+    if (factor[1] == 0.0f)
         return;
-    out[i] *= factor[0];
+    const float f = factor[0];
+    const long long stride = 4LL * gridDim.x * kThreads;
+    for (long long i = 4 * (static_cast<long long>(blockIdx.x) * kThreads + threadIdx.x); i < count; i += stride)
+    {
+        if (i + 4 <= count)
+        {
+            f4 o = *reinterpret_cast<const f4*>(out + i);
+            for (int e = 0; e < 4; e++)
+                o[e] *= f;
+            *reinterpret_cast<f4*>(out + i) = o;
+            continue;
+        }
+        for (long long k = i; k < count; k++)
+            out[k] *= f;
+    }
 }
 
 // sampler.cpp:253-263: x0 = x - bt * pred, xT = x + at * pred,
 // out = as * x0 + bs * xT (endpoint: bs = 0, as = 1 gives out = x0 exactly).
+__device__ inline float euler(float p, float x, float bt, float at, float as, float bs, int endpoint)
+{
+    const float x0 = x - bt * p;
+    if (endpoint)
+        return x0;
+    const float xT = x + at * p;
+    const float left = as * x0;
+    const float right = bs * xT;
+    return left + right;
+}
+
 __global__ __launch_bounds__(kThreads) void euler_kernel(const float* pred, const float* cur, float* out,
                                                          long long count, float bt, float at, float as, float bs,
                                                          int endpoint)
 {
-    const long long i = static_cast<long long>(blockIdx.x) * kThreads + threadIdx.x;
-    if (i >= count)
-        return;
-    const float x = cur[i];
-    const float p = pred[i];
-    const float x0 = x - bt * p;
-    if (endpoint)
+    const long long i = 4 * (static_cast<long long>(blockIdx.x) * kThreads + threadIdx.x);
+    if (i + 4 <= count)
     {
-        out[i] = x0;
+        const f4 p = *reinterpret_cast<const f4*>(pred + i);
+        const f4 x = *reinterpret_cast<const f4*>(cur + i);
+        f4 o;
+        for (int e = 0; e < 4; e++)
+            o[e] = euler(p[e], x[e], bt, at, as, bs, endpoint);
+        *reinterpret_cast<f4*>(out + i) = o;
         return;
     }
-    const float xT = x + at * p;
-    const float left = as * x0;
-    const float right = bs * xT;
-    out[i] = left + right;
+    for (long long k = i; k < count; k++)
+        out[k] = euler(pred[k], cur[k], bt, at, as, bs, endpoint);
 }
 
 int check_count(long long count, const char* what)
@@ -269,9 +326,12 @@ try
         return SV2_OK;
     if (!latent || !condition || !out)
         return set_error(SV2_EINVAL, "sv2_make_dit_input: null pointer");
-    hipLaunchKernelGGL(dit_input_kernel, dim3(blocks_for(33 * tokens)), dim3(kThreads), 0,
-                       static_cast<hipStream_t>(stream), latent, condition, out, static_cast<long long>(tokens),
-                       channel_major ? 1 : 0);
+    if (channel_major)
+        hipLaunchKernelGGL(dit_input_kernel, dim3(blocks_for_quads(33 * tokens)), dim3(kThreads), 0,
+                           static_cast<hipStream_t>(stream), latent, condition, out, static_cast<long long>(tokens));
+    else
+        hipLaunchKernelGGL(dit_input_tokens_kernel, dim3(blocks_for(33 * tokens)), dim3(kThreads), 0,
+                           static_cast<hipStream_t>(stream), latent, condition, out, static_cast<long long>(tokens));
     return launch_status("dit_input_kernel launch");
 }
 catch (...)
@@ -283,7 +343,8 @@ int64_t sv2_cfg_workspace_size(int64_t count)
 try
 {
     (void)count;
-    // partial sums of every reduction block + the factor
+    // partial sums of every reduction block (and 256 bytes kept from when the
+    // factor had a place of its own)
     return static_cast<int64_t>(sv2::kReduceBlocks) * 4 * sizeof(double) + 256;
 }
 catch (...)
@@ -306,26 +367,21 @@ try
     hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
     if (rescale == 0.0f)
     {
-        const int nb = static_cast<int>(std::min<long long>(blocks_for(count), 1LL << 20));
-        hipLaunchKernelGGL(cfg_kernel, dim3(nb), dim3(kThreads), 0, stream, positive, negative, out,
-                           static_cast<long long>(count), scale, static_cast<double*>(nullptr));
+        hipLaunchKernelGGL(cfg_kernel, dim3(blocks_for_quads(count)), dim3(kThreads), 0, stream, positive, negative,
+                           out, static_cast<long long>(count), scale);
         return launch_status("cfg_kernel launch");
     }
     if (!workspace || static_cast<int64_t>(workspace_bytes) < sv2_cfg_workspace_size(count))
         return set_error(SV2_EINVAL, "sv2_apply_cfg: the rescale needs sv2_cfg_workspace_size bytes of workspace");
     double* partial = static_cast<double*>(workspace);
-    float* factor = reinterpret_cast<float*>(static_cast<char*>(workspace) + kReduceBlocks * 4 * sizeof(double));
     const int nb = static_cast<int>(std::min<long long>(blocks_for(count), kReduceBlocks));
-    hipLaunchKernelGGL(cfg_kernel, dim3(nb), dim3(kThreads), 0, stream, positive, negative, out,
+    hipLaunchKernelGGL(cfg_sums_kernel, dim3(nb), dim3(kThreads), 0, stream, positive, negative, out,
                        static_cast<long long>(count), scale, partial);
-    if ((rc = launch_status("cfg_kernel launch")) != SV2_OK)
+    if ((rc = launch_status("cfg_sums_kernel launch")) != SV2_OK)
         return rc;
-    hipLaunchKernelGGL(cfg_factor_kernel, dim3(1), dim3(kThreads), 0, stream, partial, nb,
-                       static_cast<long long>(count), rescale, factor);
-    if ((rc = launch_status("cfg_factor_kernel launch")) != SV2_OK)
-        return rc;
-    hipLaunchKernelGGL(cfg_scale_kernel, dim3(blocks_for(count)), dim3(kThreads), 0, stream, out,
-                       static_cast<long long>(count), factor);
+    const int ns = static_cast<int>(std::min<long long>(blocks_for_quads(count), kScaleBlocks));
+    hipLaunchKernelGGL(cfg_scale_kernel, dim3(ns), dim3(kThreads), 0, stream, partial, nb, out,
+                       static_cast<long long>(count), rescale);
     return launch_status("cfg_scale_kernel launch");
 }
 catch (...)
@@ -350,7 +406,7 @@ try
     const float at = 1.0f - bt;
     const float bs = std::fmin(std::fmax(next_timestep / 1000.0f, 0.0f), 1.0f);
     const float as = 1.0f - bs;
-    hipLaunchKernelGGL(euler_kernel, dim3(blocks_for(count)), dim3(kThreads), 0, static_cast<hipStream_t>(stream),
+    hipLaunchKernelGGL(euler_kernel, dim3(blocks_for_quads(count)), dim3(kThreads), 0, static_cast<hipStream_t>(stream),
                        prediction, current, out, static_cast<long long>(count), bt, at, as, bs, 0);
     return launch_status("euler_kernel launch");
 }
@@ -373,7 +429,7 @@ try
         return set_error(SV2_EINVAL, "sv2_euler_endpoint: null pointer");
     // EulerSampler::endpoint (sampler.cpp:280-282)
     const float bt = timestep / 1000.0f;
-    hipLaunchKernelGGL(euler_kernel, dim3(blocks_for(count)), dim3(kThreads), 0, static_cast<hipStream_t>(stream),
+    hipLaunchKernelGGL(euler_kernel, dim3(blocks_for_quads(count)), dim3(kThreads), 0, static_cast<hipStream_t>(stream),
                        prediction, current, out, static_cast<long long>(count), bt, 0.0f, 1.0f, 0.0f, 1);
     return launch_status("euler_kernel launch");
 }

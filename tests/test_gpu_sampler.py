@@ -184,3 +184,23 @@ def test_sampler_loop(hip, orc, rescale):
             lat_d = s.endpoint(guided_d, lat_d, float(t))
             lat = orc.euler_endpoint(g_h, lat, float(t))
         assert np.array_equal(host(lat_d), lat)
+
+
+@pytest.mark.parametrize("count", [1, 3, 4, 5, 1023, 4097, 300001])
+@pytest.mark.parametrize("shift", [0, 1, 3])
+def test_ragged_counts_and_alignments(sampler, orc, count, shift):
+    """Counts on either side of the kernels' four-element accesses, on arrays
+    that start at any float; elements around the outputs stay untouched."""
+    print(f"[ragged] count={count} shift={shift}", flush=True)
+    pos, neg = pair((count,), count + shift)
+    box = torch.full((4, count + 8), 7.0, device="cuda")
+    p, n, o, e = (box[i, shift:shift + count] for i in range(4))
+    p.copy_(torch.from_numpy(pos))
+    n.copy_(torch.from_numpy(neg))
+    sampler.apply_cfg(p, n, 6.5, 0.0, output=o)
+    sampler.step_to(p, n, 980.0, 960.0, output=e)
+    assert np.array_equal(host(o), orc.apply_cfg(pos, neg, 6.5, 0.0))
+    assert np.array_equal(host(e), orc.euler_step(pos, neg, 980.0, 960.0))
+    sampler.apply_cfg(p, n, 6.5, 0.7, output=o)
+    within_ulps(host(o), orc.apply_cfg(pos, neg, 6.5, 0.7))
+    assert bool((box[:, :shift] == 7.0).all()) and bool((box[:, shift + count:] == 7.0).all())
