@@ -1,7 +1,8 @@
 // Matrix products of the InnerProduct layers.
 //
-// fp16 (the fast mode): hipBLASLt with fp32 accumulation.  The first product
-// of a shape on a device plans it: the library's best-ranked kernel that needs
+// fp16 (the fast mode), fp32 accumulation: gemm_mfma (gemm.hip) where
+// gemm_mfma_preferred says so, by the sizes and alignments alone; else
+// hipBLASLt.  The first library product of a shape on a device plans it: the library's best-ranked kernel that needs
 // no workspace, kept for the rest of the process.  The choice depends on the
 // shape alone, so a shape is computed with the same kernel (and rounds the
 // same way) in every process, and planning neither runs nor synchronises
@@ -237,6 +238,8 @@ int gemm_rows_gated(hipStream_t stream, int dtype, int rows, int in, int out, co
         return set_error(SV2_EUNSUPPORTED, "gemm: the gated product runs on fp16 only");
     if (rows == 0)
         return SV2_OK;
+    if (gemm_mfma_preferred(rows, in, out, kGemmResidual, x, w, nullptr, y, residual))
+        return gemm_mfma(stream, rows, in, out, x, w, nullptr, y, kGemmResidual, false, bias, gate, residual);
     const Gated g{gate, residual, bias};
     return gemm_f16(stream, rows, in, out, x, w, y, &g);
 }
@@ -256,7 +259,9 @@ int gemm_rows_bias(hipStream_t stream, int dtype, int rows, int in, int out, con
                               static_cast<float*>(y));
     if (dtype != SV2_F16)
         return set_error(SV2_EINVAL, "gemm: compute dtype must be fp32 or fp16");
-    const int rc = gemm_f16(stream, rows, in, out, x, w, y);
+    const int rc = gemm_mfma_preferred(rows, in, out, kGemmStore, x, w, nullptr, y, nullptr)
+                       ? gemm_mfma(stream, rows, in, out, x, w, nullptr, y, kGemmStore, false, nullptr, nullptr, nullptr)
+                       : gemm_f16(stream, rows, in, out, x, w, y);
     return (rc != SV2_OK || !bias) ? rc : launch_bias_rows(y, bias, SV2_F16, rows, out, stream);
 }
 

@@ -15,6 +15,7 @@
 
 using sv2::gemm_few;
 using sv2::gemm_mfma;
+using sv2::gemm_mfma_preferred;
 using sv2::gemm_rows;
 using sv2::gemm_rows_bias;
 using sv2::kGemmResidual;
@@ -364,10 +365,11 @@ int branch_mlp(const sv2_block* b, hipStream_t stream, const DevBranch& br, cons
     {
         // gate/in products with the SwiGLU gate, then the out product with
         // the gated residual (mlp_gate is the table's third row)
-        if ((rc = gemm_mfma(stream, rows, D, F, m, br.w_gate, br.w_in, g, kGemmSwiGLU, nullptr, nullptr,
+        if ((rc = gemm_mfma(stream, rows, D, F, m, br.w_gate, br.w_in, g, kGemmSwiGLU, true, nullptr, nullptr,
                             nullptr)) != SV2_OK)
             return rc;
-        return gemm_mfma(stream, rows, F, D, g, br.w_out, nullptr, out, kGemmResidual, nullptr, table + 2 * D, x);
+        return gemm_mfma(stream, rows, F, D, g, br.w_out, nullptr, out, kGemmResidual, true, nullptr, table + 2 * D,
+                         x);
     }
     if (few)
     {
@@ -377,11 +379,19 @@ int branch_mlp(const sv2_block* b, hipStream_t stream, const DevBranch& br, cons
         return gemm_few(stream, rows, F, D, g, br.w_out, nullptr, out, kGemmResidual, nullptr, table + 2 * D, x,
                         few_ws, few_bytes);
     }
-    if ((rc = gemm_rows(stream, dt, rows, D, F, m, br.w_gate, g)) != SV2_OK ||
-        (rc = gemm_rows(stream, dt, rows, D, F, m, br.w_in, u)) != SV2_OK)
+    if (dt == SV2_F16 && gemm_mfma_preferred(rows, D, F, kGemmSwiGLU, m, br.w_gate, br.w_in, g, nullptr))
+    {
+        // both products and the SwiGLU pass in one launch
+        if ((rc = gemm_mfma(stream, rows, D, F, m, br.w_gate, br.w_in, g, kGemmSwiGLU, false, nullptr, nullptr,
+                            nullptr)) != SV2_OK)
+            return rc;
+    }
+    else if ((rc = gemm_rows(stream, dt, rows, D, F, m, br.w_gate, g)) != SV2_OK ||
+             (rc = gemm_rows(stream, dt, rows, D, F, m, br.w_in, u)) != SV2_OK ||
+             (rc = sv2_swiglu(g, u, dt, static_cast<int64_t>(rows) * F, stream)) != SV2_OK)
+    {
         return rc;
-    if ((rc = sv2_swiglu(g, u, dt, static_cast<int64_t>(rows) * F, stream)) != SV2_OK)
-        return rc;
+    }
     if (dt == SV2_F16)
     {
         // the gated residual in the out product's epilogue
@@ -725,7 +735,7 @@ try
     // token RMSNorm + ada input; text skips the ada on the last layer (:1141-1151)
     if ((rc = launch_rmsnorm_table(vid, xa, dt, Lr, D, c.norm_eps, tab_va, vb.ada[0], nullptr, 1, stream)) != SV2_OK)
         return rc;
-    if ((rc = fused ? gemm_mfma(stream, Lr, D, 3 * D, xa, vb.w_qkv, nullptr, qkv_v, kGemmStore, nullptr, nullptr,
+    if ((rc = fused ? gemm_mfma(stream, Lr, D, 3 * D, xa, vb.w_qkv, nullptr, qkv_v, kGemmStore, true, nullptr, nullptr,
                                 nullptr)
                     : gemm_rows(stream, dt, Lr, D, 3 * D, xa, vb.w_qkv, qkv_v)) != SV2_OK)
         return rc;
@@ -797,7 +807,7 @@ try
     // output projections; their bias is added in the gated residual (:1180-1209)
     if (fused)
     {
-        if ((rc = gemm_mfma(stream, Lr, D, D, att_v, vb.w_proj, nullptr, p_v, kGemmResidual, vb.b_proj,
+        if ((rc = gemm_mfma(stream, Lr, D, D, att_v, vb.w_proj, nullptr, p_v, kGemmResidual, true, vb.b_proj,
                             tab_va + 2 * D, vid)) != SV2_OK)
             return rc;
     }

@@ -1,34 +1,64 @@
-// fp16 matrix products of the block's InnerProducts on gfx950 MFMA with the
-// epilogues that follow them in the block fused in (the reference runs ncnn
-// InnerProduct, seedvr2_dit_block.cpp:28-56 and :668-674, then separate
-// SwiGLU and ada-residual passes, :1093-1112 and :807-825).
+// fp16 InnerProducts of many rows on gfx950 MFMA, with the passes that follow
+// them in the block folded in (the reference runs ncnn InnerProduct,
+// seedvr2_dit_block.cpp:28-56 and :668-674, then separate SwiGLU and
+// ada-residual passes, :1093-1112 and :807-825).
 //
 //   Y[m][n] = epilogue(sum_k X[m][k] * W[n][k])      X [M][K], W [N][K] fp16
 //
-// One 256-thread workgroup computes a 256 x 256 tile of Y, one wave per
-// SIMD, each wave a 128 x 128 block as 4 x 4 MFMA tiles of 32 x 32
-// (v_mfma_f32_32x32x16_f16, 256 fp32 accumulators per lane).  K advances in
-// stages of 64 (whole 128-byte lines of every row: half-line stages halve the
-// fetch rate) through two 64 KB LDS slots.  A stage goes global -> registers
-// -> LDS: buffer loads two iterations ahead into one of two register sets,
-// then ds_write_b128 in four parts spread over the iteration before it is
-// multiplied, so the LDS writes share the bandwidth evenly with the operand
-// reads.  One barrier per stage, three quarters through it.
-// The products are computed transposed (W as the A operand), so a lane holds
-// four consecutive columns of one output row; the tile is rounded to fp16
-// (the InnerProduct's output), staged in LDS, and leaves in 16-byte row
-// segments with the epilogue applied in fp32:
-//   kStore     Y = fp16(acc)
-//   kResidual  Y = fp16((fp16(acc) + bias) * gate + R), the gated residual
-//              (bias and gate optional: without gate, Y = fp16(acc) + bias + R)
-//   kSwiGLU    two weight matrices, gate W and value W2, both [N][K]: a
-//              workgroup's 256 W rows are 128 gate rows and the same 128
-//              value rows, its output tile 256 x 128 of Y [M][N] =
-//              fp16((g / (1 + exp(-g))) * u), g, u = fp16(acc) of the halves.
-// Every fp32 operation follows the unfused kernels' order without fused
-// multiply-adds, so the epilogue adds no rounding of its own.
+// A 512-thread workgroup (8 waves, two per SIMD) computes tiles of MH x 128
+// rows by NH x 128 columns on v_mfma_f32_16x16x32_f16; a wave's part of the
+// 256 x 256 tile is 64 columns of each W half by 32 rows of each X half, 128
+// fp32 accumulators a lane.  The product is computed transposed (W as the A
+// operand), so a lane holds four consecutive columns of one output row.
+//
+// Fetch.  K moves in stages of 64 (whole 128-byte lines) through a ring of
+// LDS slots (two 64 KB, three 48 KB or four 32 KB ones), by
+// global_load_lds_dwordx4 alone: no register is held by a fetch.  A half-tile
+// of a slot is refilled as soon as the phase after the one that read it, so
+// fetches run 1.5 (256 x 256) to 3 stages ahead, and waits name the exact
+// number of younger fetches.  16-byte chunk c of row r sits in slot
+// c ^ ((r >> 1) & 7): the 16 rows an operand read takes fall on 16 different
+// bank groups.
+//
+// Phases.  A stage is walked in quadrants (W half x X half), each a memory
+// part (operand reads, fetches, waits) and 16 MFMAs, with a barrier after
+// each.  The two waves of a SIMD belong to different groups, one slot apart:
+// one group multiplies while the other one reads.
+//
+// Workgroups are persistent (one per CU) and take tiles in XCD-contiguous
+// runs; the ring runs on across tiles, so a tile's first stages are in flight
+// during the epilogue of the one before.  Outputs leave with non-temporal
+// stores: written through the L2 they evict the operand panels (128 KB a tile
+// and CU is the whole L2 of an XCD), qkv at 21658 rows 758 us against 667.
+//
+// What bounds it, 21658 rows (MI355X; the library product beside it):
+//   qkv 2560 -> 7680                   594 us (1.43 PFLOP/s)   589
+//   proj 2560 -> 2560 + residual       250 us                  276 (its residual apart)
+//   gate/in 2560 -> 2 x 6912 + SwiGLU  1062 us                 1067 + 137
+//   out 6912 -> 2560 + residual        605 us                  676 (its residual apart)
+// With all-zero operands the same launches take 434 / 215 / 773 / 512 us: on
+// random data the clock drops under the matrix cores' power, and the rest is
+// LDS bandwidth (192 KB of operand reads and 64 KB of fetch a 256 x 256 stage,
+// 2048 cycles at 128 B/clk, as many as its MFMAs take).  A 128 x 128 tile
+// reads three bytes of LDS where the large one reads two, and runs at 0.39 us
+// a stage against 0.24 us for a quarter of the large one's; it is there for
+// the products that would leave CUs idle.  `KS` is the 128 x 128 tile with a
+// 64 x 64 part per wave: the two groups take one k-step of each stage each and
+// add their sums at the end (reads a third less LDS than 64 x 32 parts do).
+//
+// Epilogues, in fp32 from the accumulators:
+//   kGemmStore     Y = fp16(acc)
+//   kGemmResidual  Y = fp16(acc * gate + R + bias), one rounding; `rounded`:
+//                  fp16((fp16(acc) + bias) * gate + R), the unfused passes'
+//                  order (gate and bias optional)
+//   kGemmSwiGLU    two weight matrices, gate W and value W2, both [N][K]: the
+//                  W halves of a tile are the gate and value rows of the same
+//                  128 columns, Y = fp16(g / (1 + exp(-g)) * u); `rounded`: g
+//                  and u rounded to fp16 first, as the separate products are
 #include "sv2_internal.h"
+#include <algorithm>
 #include <climits>
+#include <type_traits>
 
 #pragma clang fp contract(off)
 
@@ -39,130 +69,104 @@ namespace
 
 typedef __attribute__((ext_vector_type(8))) _Float16 h8;
 typedef __attribute__((ext_vector_type(4))) _Float16 h4;
-typedef __attribute__((ext_vector_type(16))) float f16acc;
+typedef __attribute__((ext_vector_type(4))) float f4;
+typedef __attribute__((ext_vector_type(4), aligned(4))) float f4u; // gate and bias: any float alignment
+typedef __attribute__((ext_vector_type(4))) unsigned u4;
 
-constexpr int kBM = 256;                      // rows of Y per workgroup
-constexpr int kBN = 256;                      // columns of Y (rows of W) per workgroup
-constexpr int kBK = 64;                       // K per stage: whole 128-byte lines of every row
-constexpr int kKSteps = kBK / 16;             // MFMA k-steps per stage
-constexpr int kRowBytes = kBK * 2;            // 128
-constexpr int kTileBytes = kBM * kRowBytes;   // 32 KB: one operand tile of a stage
-constexpr int kStageBytes = 2 * kTileBytes;   // 64 KB: W tile + X tile
-constexpr int kThreads = 256;                 // 4 waves, one per SIMD, 128 x 128 of Y each
-constexpr int kGroupM = 4;                    // row bands per tile group (see the tile order)
-constexpr int kEpiStride = 272;               // bytes per staged output row (256 + 16: bank spread)
-constexpr int kEpiBytes = 128 * kEpiStride;   // one wave's 128 x 128 fp16 block
-constexpr int kLds = (2 * kStageBytes > 4 * kEpiBytes) ? 2 * kStageBytes : 4 * kEpiBytes;
-static_assert(kLds <= 160 * 1024, "LDS of one gfx950 CU");
+constexpr int kThreads = 512;      // 8 waves, two per SIMD
+constexpr int kHalf = 128;         // rows of one operand half-tile
+constexpr int kBK = 64;            // K per stage: whole 128-byte lines of every row
+constexpr int kRowBytes = kBK * 2; // 128
+constexpr int kHalfBytes = kHalf * kRowBytes; // 16 KB
+constexpr int kEpiWave = 16 * 128; // bytes of one wave's epilogue staging: 16 rows of 64 fp16
+constexpr int kEpiBytes = 8 * kEpiWave;
+constexpr int kMaxLds = 160 * 1024;
+constexpr int kCus = 256;            // compute units of one MI355X
+constexpr int kPreferRows = 256;
+constexpr int kTouchAhead = 3;      // stages before a tile's end
+constexpr float kLog2e = 1.4426950408889634f;
 
-constexpr int kStore = kGemmStore;
-constexpr int kResidual = kGemmResidual;
-constexpr int kSwiGLU = kGemmSwiGLU;
-
-struct GemmArgs
+struct TileArgs
 {
     const _Float16* x;  // [M][K]
     const _Float16* w;  // [N][K]
-    const _Float16* w2; // kSwiGLU: the value projection [N][K]
+    const _Float16* w2; // SwiGLU: the value projection [N][K]
     _Float16* y;        // [M][N]
-    const _Float16* r;  // kResidual: [M][N]
+    const _Float16* r;  // residual [M][N]
     const float* bias;  // [N] or null
     const float* gate;  // [N] or null
     int m, n, k;
-    int epi;
-    int tiles_n;        // N / 256 (kSwiGLU: N / 128)
+    int rounded;        // the product is rounded to fp16 before the epilogue
+    int tiles_m;        // row bands
+    int tiles_n;        // column tiles
+    int total;          // tiles_m * tiles_n
+    int group_m;        // row bands per tile group
 };
 
-// Global -> register -> LDS staging.  Lane l of wave w loads rows
-// 64 w + 8 i + l / 8 (i = 0..7) of the W tile and of the X tile, 16-byte
-// chunk l % 8 of the stage's 128 bytes, and writes it to slot
-// (l % 8) ^ (row % 8) of its row.  Buffer loads: the lane's part of the
-// offset is one VGPR per operand, the row and stage parts are uniform (SGPR
-// offset); X rows past M lie past the buffer's end and read as zero.
-struct Operands
+// Stages an operand tile of MH (X) + NH (W) halves takes, and how many of
+// them fit in LDS beside the epilogue staging.
+template <int MH, int NH>
+struct Shape
 {
-    __amdgpu_buffer_rsrc_t w;
-    __amdgpu_buffer_rsrc_t x;
-    int vw;   // lane's byte offset in W: (wrow0 + 64 wave + lane / 8) * 2K + 16 (lane % 8)
-    int vx;   // lane's byte offset in X: (m0 + 64 wave + lane / 8) * 2K + 16 (lane % 8)
-    int row8; // bytes of 8 rows: 16 K
+    static constexpr int kStageBytes = (MH + NH) * kHalfBytes;
+    static constexpr int kFit = (kMaxLds - kEpiBytes) / kStageBytes;
+    static constexpr int kSlots = kFit > 4 ? 4 : kFit;
+    static constexpr int kLds = kSlots * kStageBytes + kEpiBytes;
+    static_assert(kSlots >= 2 && kLds <= kMaxLds, "LDS of one gfx950 CU");
 };
 
-struct StageRegs
+// 16 bytes per lane from global memory (uniform base + 32-bit lane offset)
+// straight into LDS at lds + 16 * lane (lds wave-uniform, in M0; one wait
+// state between the write of M0 and its use).  The compiler does not count
+// these loads in its vmcnt waits; the loop waits for them itself.
+__device__ inline void dma16(const char* base, unsigned voff, unsigned lds)
 {
-    uint4 w[8];
-    uint4 x[8];
-};
-
-__device__ inline Operands make_operands(const GemmArgs& a, int m0, int wbase, int wave, int lane)
-{
-    Operands o;
-    const bool swiglu = a.epi == kSwiGLU;
-    const _Float16* wsrc = swiglu && wave >= 2 ? a.w2 : a.w;
-    const int wrow0 = swiglu ? wbase - 128 * (wave >> 1) : wbase;
-    o.w = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16*>(wsrc), static_cast<short>(0), a.n * a.k * 2,
-                                            0x00020000);
-    o.x = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16*>(a.x), static_cast<short>(0), a.m * a.k * 2,
-                                            0x00020000);
-    // byte offsets in 32-bit unsigned arithmetic: the rows of the last, padded
-    // X tile reach round_up(m, kBM) - 1, whose offset can pass INT_MAX when m *
-    // k * 2 is just under it; it stays below 2^32 (k < 2^22), and the buffer
-    // resource returns zeros for any offset past the operand
-    const uint32_t row = 64u * static_cast<uint32_t>(wave) + static_cast<uint32_t>(lane >> 3);
-    const uint32_t kb = 2u * static_cast<uint32_t>(a.k);
-    o.vw = static_cast<int>((static_cast<uint32_t>(wrow0) + row) * kb + 16u * static_cast<uint32_t>(lane & 7));
-    o.vx = static_cast<int>((static_cast<uint32_t>(m0) + row) * kb + 16u * static_cast<uint32_t>(lane & 7));
-    o.row8 = 16 * a.k;
-    return o;
+    const unsigned long long b = reinterpret_cast<unsigned long long>(base);
+    const unsigned lo = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(b));
+    const unsigned hi = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(b >> 32));
+    lds = __builtin_amdgcn_readfirstlane(lds);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :
+                 : "s"(lds), "v"(voff), "s"(static_cast<unsigned long long>(hi) << 32 | lo)
+                 : "memory", "m0");
 }
 
-__device__ inline void load_stage(const Operands& o, StageRegs& r, int kt)
+// The same with 4 bytes per lane, for its effect on the L2 alone: lds is a
+// 256-byte sink.
+__device__ inline void touch(const void* p, unsigned lds)
 {
-    const int k0 = kt * kRowBytes;
-#pragma unroll
-    for (int i = 0; i < 8; i++)
-    {
-        const int so = __builtin_amdgcn_readfirstlane(i * o.row8 + k0);
-        r.w[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(o.w, o.vw, so, 0));
-        r.x[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(o.x, o.vx, so, 0));
-    }
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
+                 :
+                 : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(p)
+                 : "memory", "m0");
 }
 
-__device__ inline void store_stage(const StageRegs& r, char* stage, int wave, int lane)
+template <int N>
+__device__ inline void wait_vm()
 {
-#pragma unroll
-    for (int i = 0; i < 8; i++)
-    {
-        const int row = 64 * wave + 8 * i + (lane >> 3);
-        const int off = row * kRowBytes + (((lane & 7) ^ (row & 7)) << 4);
-        *reinterpret_cast<uint4*>(stage + off) = r.w[i];
-        *reinterpret_cast<uint4*>(stage + kTileBytes + off) = r.x[i];
-    }
+    static_assert(N >= 0 && N < 64, "vmcnt holds 6 bits");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// part p of a stage: the lane's W and X rows of groups i = 2p, 2p + 1
-__device__ inline void load_part(const Operands& o, StageRegs& r, int kt, int p)
+__device__ inline void wait_lds()
 {
-    const int k0 = kt * kRowBytes;
-#pragma unroll
-    for (int i = 2 * p; i < 2 * p + 2; i++)
-    {
-        const int so = __builtin_amdgcn_readfirstlane(i * o.row8 + k0);
-        r.w[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(o.w, o.vw, so, 0));
-        r.x[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(o.x, o.vx, so, 0));
-    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 }
 
-__device__ inline void store_part(const StageRegs& r, char* stage, int wave, int lane, int p)
+// A wave's LDS operations complete in order; this keeps the compiler from
+// reordering them.
+__device__ inline void lds_order()
 {
-#pragma unroll
-    for (int i = 2 * p; i < 2 * p + 2; i++)
-    {
-        const int row = 64 * wave + 8 * i + (lane >> 3);
-        const int off = row * kRowBytes + (((lane & 7) ^ (row & 7)) << 4);
-        *reinterpret_cast<uint4*>(stage + off) = r.w[i];
-        *reinterpret_cast<uint4*>(stage + kTileBytes + off) = r.x[i];
-    }
+    asm volatile("" ::: "memory");
+}
+
+// A workgroup barrier without the waits of __syncthreads (the fetches in
+// flight stay in flight); nothing is scheduled across it.
+__device__ inline void bar()
+{
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
 }
 
 __device__ inline float h2f(_Float16 v)
@@ -170,314 +174,760 @@ __device__ inline float h2f(_Float16 v)
     return static_cast<float>(v);
 }
 
-struct EpiCols
+__device__ inline float round16(float v)
 {
-    float b[8];
-    float g[8];
-};
+    return static_cast<float>(static_cast<_Float16>(v));
+}
 
-__device__ inline EpiCols epi_cols(const GemmArgs& a, int col)
+// Tile id -> (row band, column tile): groups of group_m row bands, the bands
+// of one column of tiles first.
+__device__ inline void tile_at(const TileArgs& a, int id, int* tm, int* tn)
 {
-    EpiCols c;
-#pragma unroll
-    for (int e = 0; e < 8; e++)
+    const int per = a.group_m * a.tiles_n;
+    const int grp = id / per;
+    const int first = grp * a.group_m;
+    const int rows = min(a.group_m, a.tiles_m - first);
+    const int in = id - grp * per;
+    *tn = in / rows;
+    *tm = first + (in - *tn * rows);
+}
+
+// Waits until at most n fetches are outstanding; n one of the counts the
+// pipeline's start and end meet (any other waits for all of them).
+__device__ inline void wait_younger(int n)
+{
+    switch (n)
     {
-        c.b[e] = 0.f;
-        c.g[e] = 1.f;
+    case 18: wait_vm<18>(); break;
+    case 16: wait_vm<16>(); break;
+    case 14: wait_vm<14>(); break;
+    case 12: wait_vm<12>(); break;
+    case 8: wait_vm<8>(); break;
+    case 6: wait_vm<6>(); break;
+    case 4: wait_vm<4>(); break;
+    default: wait_vm<0>(); break;
     }
-    if (a.epi == kResidual)
-    {
+}
+
+// Rounds and stores one wave's part of a tile: for W half h and X half j the
+// lane holds rows row0 + 128 j + 16 b + lane % 16, columns col0 + 128 h +
+// 16 t + 4 (lane / 16) .. + 3 of acc[h][j][t][b].  16 rows x 64 columns at a
+// time go through `mine` (2 KB of LDS, this wave's own), 16-byte chunk c of
+// row r in slot c ^ (r & 7), so that residual rows are read and output rows
+// written as whole 128-byte lines.
+template <int MH, int NH, int EPI>
+__device__ __forceinline__ void epilogue(const TileArgs& a, f4 (&acc)[NH][MH][4][2], char* mine, int row0, int col0, int lane)
+{
+    constexpr bool kSw = EPI == kGemmSwiGLU;
+    const int lr = lane & 15;
+    const int lq = lane >> 4;
+    const int rr = lane >> 3; // rows rr, rr + 8 of the line accesses
+    const int cc = lane & 7;
+    char* line[2];
+    char* quad[4];
 #pragma unroll
-        for (int e = 0; e < 8; e++)
+    for (int s = 0; s < 2; s++)
+        line[s] = mine + (rr + 8 * s) * 128 + ((cc ^ (rr & 7)) << 4);
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+        quad[t] = mine + lr * 128 + (((2 * t + (lq >> 1)) ^ (lr & 7)) << 4) + 8 * (lq & 1);
+#pragma unroll
+    for (int h = 0; h < (kSw ? 1 : NH); h++)
+    {
+        const int col = col0 + kHalf * h;
+        f4 gate[4], bias[4];
+        u4 res[MH][2][2];
+        if constexpr (EPI == kGemmResidual)
         {
-            if (a.bias)
-                c.b[e] = a.bias[col + e];
-            if (a.gate)
-                c.g[e] = a.gate[col + e];
+#pragma unroll
+            for (int j = 0; j < MH; j++)
+#pragma unroll
+                for (int b = 0; b < 2; b++)
+#pragma unroll
+                    for (int s = 0; s < 2; s++)
+                    {
+                        const int row = min(row0 + kHalf * j + 16 * b + rr + 8 * s, a.m - 1);
+                        res[j][b][s] = __builtin_nontemporal_load(
+                            reinterpret_cast<const u4*>(a.r + static_cast<long long>(row) * a.n + col + 8 * cc));
+                    }
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+            {
+                gate[t] = f4{1.f, 1.f, 1.f, 1.f};
+                bias[t] = f4{0.f, 0.f, 0.f, 0.f};
+                if (a.gate)
+                    gate[t] = *reinterpret_cast<const f4u*>(a.gate + col + 16 * t + 4 * lq);
+                if (a.bias)
+                    bias[t] = *reinterpret_cast<const f4u*>(a.bias + col + 16 * t + 4 * lq);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < MH; j++)
+        {
+#pragma unroll
+            for (int b = 0; b < 2; b++)
+            {
+                h4 old[4];
+                if constexpr (EPI == kGemmResidual)
+                {
+                    *reinterpret_cast<u4*>(line[0]) = res[j][b][0];
+                    *reinterpret_cast<u4*>(line[1]) = res[j][b][1];
+                    lds_order();
+#pragma unroll
+                    for (int t = 0; t < 4; t++)
+                        old[t] = *reinterpret_cast<const h4*>(quad[t]);
+                    lds_order();
+                }
+#pragma unroll
+                for (int t = 0; t < 4; t++)
+                {
+                    h4 o;
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                    {
+                        float v = acc[h][j][t][b][e];
+                        if constexpr (kSw)
+                        {
+                            // silu(g) u: exp2 and the reciprocal, each within
+                            // an fp32 ulp, in place of expf and a divide (about
+                            // 45 instructions an element, 1197 us against 1074
+                            // for gate/in at 21658 rows)
+                            float u = acc[NH - 1][j][t][b][e];
+                            if (a.rounded)
+                            {
+                                v = round16(v);
+                                u = round16(u);
+                            }
+                            const float den = 1.f + __builtin_amdgcn_exp2f(v * -kLog2e);
+                            v = v * __builtin_amdgcn_rcpf(den) * u;
+                        }
+                        if constexpr (EPI == kGemmResidual)
+                        {
+                            const float r = h2f(old[t][e]);
+                            if (!a.rounded)
+                            {
+                                v = v * gate[t][e] + r + bias[t][e];
+                            }
+                            else
+                            {
+                                v = round16(v);
+                                if (a.bias)
+                                    v = v + bias[t][e];
+                                if (a.gate)
+                                    v = v * gate[t][e];
+                                v = v + r;
+                            }
+                        }
+                        o[e] = static_cast<_Float16>(v);
+                    }
+                    *reinterpret_cast<h4*>(quad[t]) = o;
+                }
+                lds_order();
+#pragma unroll
+                for (int s = 0; s < 2; s++)
+                {
+                    const int row = row0 + kHalf * j + 16 * b + rr + 8 * s;
+                    const u4 v = *reinterpret_cast<const u4*>(line[s]);
+                    if (row < a.m)
+                        __builtin_nontemporal_store(v, reinterpret_cast<u4*>(a.y + static_cast<long long>(row) * a.n + col + 8 * cc));
+                }
+                lds_order();
+            }
         }
     }
-    return c;
 }
 
-__device__ inline h8 finish_segment(const GemmArgs& a, const EpiCols& c, const h8 p, long long row, int col)
-{
-    h8 out;
-    if (a.epi == kStore)
-        return p;
-    const h8 res = *reinterpret_cast<const h8*>(a.r + row * a.n + col);
-#pragma unroll
-    for (int e = 0; e < 8; e++)
-    {
-        float v = h2f(p[e]);
-        if (a.bias)
-            v = v + c.b[e];
-        if (a.gate)
-            v = v * c.g[e];
-        v = v + h2f(res[e]);
-        out[e] = static_cast<_Float16>(v);
-    }
-    return out;
-}
-
-__global__ __launch_bounds__(kThreads) void gemm_f16_kernel(GemmArgs a)
+template <int MH, int NH, int EPI, bool KS>
+__global__ __launch_bounds__(kThreads) void gemm_tile_kernel(TileArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) char smem[];
+    using S = Shape<MH, NH>;
+    constexpr int kSlots = S::kSlots;
+    constexpr int kFour = MH == 2 && NH == 2; // four phases a stage
+    static_assert(!KS || MH + NH == 2, "the K-split form is the 128 x 128 one");
+    constexpr int kSteps = KS ? 1 : 2; // k-steps of 32 a wave multiplies per stage
+    constexpr int kXT = KS ? 4 : 2;    // 16-row X tiles of a wave and half
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lr = lane & 31;
-    const int g = lane >> 5;
-    const int wm = wave >> 1; // 128-row half of the tile (X rows)
-    const int wn = wave & 1;  // 128-column half (W rows)
-
-    // workgroup ids go round-robin over the 8 XCDs; each XCD takes a
-    // contiguous run of tiles (whole row bands, sharing their X rows in the
-    // XCD's L2): XCD x owns tiles [x q + min(x, r), ...) for total = 8 q + r
-    const int total = static_cast<int>(gridDim.x);
-    const int xcd = blockIdx.x & 7;
-    const int q8 = total >> 3;
-    const int r8 = total & 7;
-    const int id = xcd * q8 + min(xcd, r8) + static_cast<int>(blockIdx.x >> 3);
-    // grouped order: consecutive ids walk kGroupM row bands of one column of
-    // tiles before the next column, so the workgroups an XCD runs at once
-    // cover about 4 row bands x 8 column tiles and share both operands in L2
-    const int tiles_m = (a.m + kBM - 1) / kBM;
-    const int per_group = kGroupM * a.tiles_n;
-    const int grp = id / per_group;
-    const int first_m = grp * kGroupM;
-    const int group_rows = min(kGroupM, tiles_m - first_m);
-    const int in_group = id - grp * per_group;
-    const int tm = first_m + in_group % group_rows;
-    const int tn = in_group / group_rows;
-    const int m0 = tm * kBM;
-    const bool swiglu = a.epi == kSwiGLU;
-    const int n0 = swiglu ? tn * 128 : tn * kBN;
+    const int grp = wave >> 2; // the two groups alternate
+    // rows of the wave's part in each W half and X half.  KS: the groups share
+    // a 64 x 64 part and take one k-step of a stage each
+    const int wrow = KS ? 64 * (wave & 1) : 64 * grp;
+    const int xrow = KS ? 64 * ((wave >> 1) & 1) : 32 * (wave & 3);
+    const int lr = lane & 15;
+    const int lq = lane >> 4;
     const int nk = a.k / kBK;
+    const unsigned k2 = 2u * static_cast<unsigned>(a.k);
 
-    // per-lane operand offsets: row 128 * wn (W) / 128 * wm (X) + lr of a
-    // tile, chunk 2 ks + g; the 32-row blocks add 4096 bytes each
-    const int swz = lr & 7;
-    int offw[kKSteps];
-    int offx[kKSteps];
-#pragma unroll
-    for (int ks = 0; ks < kKSteps; ks++)
-    {
-        offw[ks] = (128 * wn + lr) * kRowBytes + (((2 * ks + g) ^ swz) << 4);
-        offx[ks] = kTileBytes + (128 * wm + lr) * kRowBytes + (((2 * ks + g) ^ swz) << 4);
-    }
-
-    f16acc acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-            acc[i][j] = f16acc{};
-
-    const Operands ops = make_operands(a, m0, n0, wave, lane);
-    // Stage s: loaded into register set s % 2 two iterations ahead, written
-    // to LDS slot s % 2 in four parts (part 0 after the barrier of iteration
-    // s - 2, parts 1-3 during the first three k-steps of iteration s - 1,
-    // each part's registers reloaded with stage s + 2 right after), read
-    // after the barrier of iteration s - 1.  Every iteration writes and
-    // loads (stages past the last load stage nk - 1 again and are never
-    // multiplied), so the loop body has no branches and the compiler's waits
-    // for the loads are exact.
-    StageRegs ra, rb;
-    const int last = nk - 1;
-    load_stage(ops, ra, 0);
-    load_stage(ops, rb, min(1, last));
-    store_stage(ra, smem, wave, lane);
-    load_stage(ops, ra, min(2, last));
-    store_part(rb, smem + kStageBytes, wave, lane, 0);
-    load_part(ops, rb, min(3, last), 0);
-    __syncthreads();
-
-    h8 fw[2][4], fx[2][4];
-    auto read_ops = [&](h8 (&w4)[4], h8 (&x4)[4], const char* st, int ks) {
-#pragma unroll
-        for (int b = 0; b < 4; b++)
-        {
-            w4[b] = *reinterpret_cast<const h8*>(st + offw[ks] + b * 4096);
-            x4[b] = *reinterpret_cast<const h8*>(st + offx[ks] + b * 4096);
-        }
-    };
-    auto mfmas = [&](const h8 (&w4)[4], const h8 (&x4)[4]) {
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w4[j], x4[i], acc[i][j], 0, 0, 0);
-    };
-    // scheduling groups (masks: 0x100 LDS read, 0x008 MFMA, 0x200 LDS write,
-    // 0x020 global read): a phase's eight operand reads first, then its 16
-    // MFMAs in groups of four, each group's first MFMA followed by one write
-    // and one load
-    auto interleave = [&]() {
-#pragma unroll
-        for (int m = 0; m < 4; m++)
-        {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
-        }
-    };
-    read_ops(fw[0], fx[0], smem, 0);
-
-    // Iteration kt (stage kt in slot kt % 2, its k-step 0 operands in
-    // fw/fx[0]; `nx` holds stage kt + 1's parts 1-3, `cur` stage kt + 2):
-    // k-steps 0-2 each with the next k-step's reads and one part of stage
-    // kt + 1; the barrier (the slot's reads are done, stage kt + 1 is
-    // visible); k-step 3 with stage kt + 1's first reads and part 0 of stage
-    // kt + 2 into this slot.
-    auto iter = [&](int kt, StageRegs& cur, StageRegs& nx) {
-        char* st = smem + (kt & 1) * kStageBytes;
-        char* sn = smem + ((kt + 1) & 1) * kStageBytes;
-#pragma unroll
-        for (int ks = 0; ks < kKSteps - 1; ks++)
-        {
-            read_ops(fw[(ks + 1) & 1], fx[(ks + 1) & 1], st, ks + 1);
-            mfmas(fw[ks & 1], fx[ks & 1]);
-            store_part(nx, sn, wave, lane, ks + 1);
-            load_part(ops, nx, min(kt + 3, last), ks + 1);
-            __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
-            interleave();
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        __syncthreads();
-        read_ops(fw[0], fx[0], sn, 0);
-        mfmas(fw[1], fx[1]);
-        store_part(cur, st, wave, lane, 0);
-        load_part(ops, cur, min(kt + 4, last), 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
-        interleave();
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    int kt = 0;
-    for (; kt + 1 < nk; kt += 2)
-    {
-        iter(kt, ra, rb);
-        iter(kt + 1, rb, ra);
-    }
-    if (kt < nk)
-        iter(kt, ra, rb);
-
-    // acc[i][j] register 4q + e holds Y row m0 + 128 wm + 32 i + lr, column
-    // n0 + 128 wn + 32 j + 8 q + 4 g + e.
-    __syncthreads();
-    char* mine = smem + wave * kEpiBytes;
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-#pragma unroll
-            for (int q = 0; q < 4; q++)
-            {
-                h4 v;
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                    v[e] = static_cast<_Float16>(acc[i][j][4 * q + e]);
-                *reinterpret_cast<h4*>(mine + (32 * i + lr) * kEpiStride + (32 * j + 8 * q + 4 * g) * 2) = v;
-            }
-
-    if (swiglu)
-    {
-        // gate block: wave (wm, 0), value block: wave (wm, 1); wave (wm, wn)
-        // writes rows 64 wn..64 wn + 63 of the 128-row half wm
-        __syncthreads();
-        const char* gate_blk = smem + (2 * wm) * kEpiBytes;
-        const char* val_blk = smem + (2 * wm + 1) * kEpiBytes;
-        const int chunk = lane & 15;
-        const int ycol = n0 + 8 * chunk;
-#pragma unroll 4
-        for (int it = 0; it < 16; it++)
-        {
-            const int rl = 64 * wn + 4 * it + (lane >> 4);
-            const long long row = m0 + 128 * wm + rl;
-            if (row >= a.m)
-                continue;
-            const h8 gv = *reinterpret_cast<const h8*>(gate_blk + rl * kEpiStride + chunk * 16);
-            const h8 uv = *reinterpret_cast<const h8*>(val_blk + rl * kEpiStride + chunk * 16);
-            h8 out;
-#pragma unroll
-            for (int e = 0; e < 8; e++)
-            {
-                const float gf = h2f(gv[e]);
-                const float den = 1.f + expf(-gf);
-                out[e] = static_cast<_Float16>((gf / den) * h2f(uv[e]));
-            }
-            *reinterpret_cast<h8*>(a.y + row * a.n + ycol) = out;
-        }
+    // tile list of this workgroup: round r gives XCD x the contiguous ids
+    // [r G + x G/8, + G/8), the last round an even share of what is left
+    const int G = static_cast<int>(gridDim.x);
+    const int per_xcd = G >> 3;
+    const int xcd = blockIdx.x & 7;
+    const int local = blockIdx.x >> 3;
+    const int full = a.total / G;
+    const int left = a.total - full * G;
+    const int left_per = (left + 7) >> 3;
+    const int left_id = xcd * left_per + local;
+    const bool has_left = local < left_per && left_id < left;
+    const int ntiles = full + (has_left ? 1 : 0);
+    if (ntiles == 0)
         return;
-    }
+    auto tile_of = [&](int i, int* m0, int* n0) {
+        const int id = i < full ? i * G + xcd * per_xcd + local : full * G + left_id;
+        int tm, tn;
+        tile_at(a, id, &tm, &tn);
+        *m0 = tm * (kHalf * MH);
+        *n0 = tn * (EPI == kGemmSwiGLU ? kHalf : kHalf * NH);
+    };
 
-    __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0)
-    __builtin_amdgcn_wave_barrier();
-    const int chunk = lane & 15;
-    const int col = n0 + 128 * wn + 8 * chunk;
-    const EpiCols ec = epi_cols(a, col);
-#pragma unroll 4
-    for (int it = 0; it < 32; it++)
+    // fetch side: this wave fetches rows 16 wave + 8 i + lane / 8 of every
+    // half-tile; the lane's LDS slot lane & 7 of the row holds chunk
+    // (lane & 7) ^ ((row >> 1) & 7)
+    const unsigned frow = 16u * wave + (lane >> 3);
+    const unsigned chunk0 = 16u * ((lane & 7) ^ (lane >> 4));
+    const unsigned vw0 = frow * k2 + chunk0;
+    const unsigned vw1 = (frow + 8) * k2 + (chunk0 ^ 64u);
+    unsigned vx[MH][2];
+    const char* fx = nullptr;       // X rows of the tile being fetched, at the stage being fetched
+    const char* fw[NH];
+    int f_tile = -1;                // tile being fetched
+    int f_kt = nk;                  // next stage to fetch of it (nk: open the next tile)
+    unsigned f_slot = 0;
+    auto open_tile = [&]() {
+        f_tile++;
+        f_kt = 0;
+        int m0, n0;
+        tile_of(f_tile, &m0, &n0);
+        fx = reinterpret_cast<const char*>(a.x) + static_cast<unsigned long long>(m0) * k2;
+        const int lastrow = a.m - 1 - m0;
+#pragma unroll
+        for (int j = 0; j < MH; j++)
+        {
+            // rows past M repeat the last one; their sums are never stored
+            vx[j][0] = static_cast<unsigned>(min(static_cast<int>(kHalf * j + frow), lastrow)) * k2 + chunk0;
+            vx[j][1] = static_cast<unsigned>(min(static_cast<int>(kHalf * j + frow + 8), lastrow)) * k2 + (chunk0 ^ 64u);
+        }
+#pragma unroll
+        for (int h = 0; h < NH; h++)
+        {
+            const _Float16* src = (EPI == kGemmSwiGLU && h == 1) ? a.w2 : a.w;
+            const int row = (EPI == kGemmSwiGLU) ? n0 : n0 + kHalf * h;
+            fw[h] = reinterpret_cast<const char*>(src) + static_cast<unsigned long long>(row) * k2;
+        }
+    };
+    const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<size_t>(smem));
+    const unsigned lds_wave = lds0 + 16u * wave * kRowBytes;
+    auto fetch_w = [&](int h) {
+        const unsigned d = lds_wave + f_slot + h * kHalfBytes;
+        dma16(fw[h], vw0, d);
+        dma16(fw[h], vw1, d + 8 * kRowBytes);
+    };
+    auto fetch_x = [&](int j) {
+        const unsigned d = lds_wave + f_slot + (NH + j) * kHalfBytes;
+        dma16(fx, vx[j][0], d);
+        dma16(fx, vx[j][1], d + 8 * kRowBytes);
+    };
+    // moves the fetch side to the next stage (of the next tile when needed)
+    auto fetch_next = [&]() {
+        f_kt++;
+        f_slot = f_slot + S::kStageBytes == kSlots * S::kStageBytes ? 0u : f_slot + S::kStageBytes;
+        fx += kRowBytes;
+#pragma unroll
+        for (int h = 0; h < NH; h++)
+            fw[h] += kRowBytes;
+        if (f_kt == nk && f_tile + 1 < ntiles)
+            open_tile();
+    };
+
+    // operand reads: row wrow + 16 t + lr (W) / xrow + 16 b + lr (X) of a
+    // half, chunk 4 ks + lq, in slot chunk ^ ((row >> 1) & 7)
+    const unsigned swz = (lr >> 1) & 7;
+    unsigned ow[kSteps], ox[kSteps];
+#pragma unroll
+    for (int ks = 0; ks < kSteps; ks++)
     {
-        const int rl = 4 * it + (lane >> 4);
-        const long long row = m0 + 128 * wm + rl;
-        if (row >= a.m)
-            continue;
-        const h8 p = *reinterpret_cast<const h8*>(mine + rl * kEpiStride + chunk * 16);
-        *reinterpret_cast<h8*>(a.y + row * a.n + col) = finish_segment(a, ec, p, row, col);
+        const unsigned c = ((4 * (KS ? grp : ks) + lq) ^ swz) << 4;
+        ow[ks] = (wrow + lr) * kRowBytes + c;
+        ox[ks] = NH * kHalfBytes + (xrow + lr) * kRowBytes + c;
+    }
+    h8 rw[kSteps][4];
+    h8 rx[MH][kSteps][kXT];
+    f4 acc[NH][MH][4][kXT];
+    unsigned r_slot = 0;
+    auto read_w = [&](int h) {
+        const char* st = smem + r_slot + h * kHalfBytes;
+#pragma unroll
+        for (int ks = 0; ks < kSteps; ks++)
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+                rw[ks][t] = *reinterpret_cast<const h8*>(st + ow[ks] + t * 16 * kRowBytes);
+    };
+    auto read_x = [&](int j) {
+        const char* st = smem + r_slot + j * kHalfBytes;
+#pragma unroll
+        for (int ks = 0; ks < kSteps; ks++)
+#pragma unroll
+            for (int b = 0; b < kXT; b++)
+                rx[j][ks][b] = *reinterpret_cast<const h8*>(st + ox[ks] + b * 16 * kRowBytes);
+    };
+    auto mma = [&](int h, int j) {
+#pragma unroll
+        for (int ks = 0; ks < kSteps; ks++)
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int b = 0; b < kXT; b++)
+                    acc[h][j][t][b] =
+                        __builtin_amdgcn_mfma_f32_16x16x32_f16(rw[ks][t], rx[j][ks][b], acc[h][j][t][b], 0, 0, 0);
+    };
+
+    auto read_slot_next = [&]() {
+        r_slot = r_slot + S::kStageBytes == kSlots * S::kStageBytes ? 0u : r_slot + S::kStageBytes;
+    };
+    auto clear = [&]() {
+#pragma unroll
+        for (int h = 0; h < NH; h++)
+#pragma unroll
+            for (int j = 0; j < MH; j++)
+#pragma unroll
+                for (int t = 0; t < 4; t++)
+#pragma unroll
+                    for (int b = 0; b < kXT; b++)
+                        acc[h][j][t][b] = f4{0.f, 0.f, 0.f, 0.f};
+    };
+
+    // the first kSlots stages
+    const int stages = ntiles * nk;
+    open_tile();
+#pragma unroll
+    for (int s = 0; s < kSlots; s++)
+        if (s < stages)
+        {
+            fetch_w(0);
+            fetch_x(0);
+            if constexpr (MH == 2)
+                fetch_x(1);
+            if constexpr (NH == 2)
+                fetch_w(1);
+            fetch_next();
+        }
+    // stage 0 has landed once only the younger stages' fetches are outstanding
+    constexpr int kPer = 2 * (MH + NH); // fetches per wave and stage
+    wait_younger(min(stages - 1, kSlots - 1) * kPer);
+    bar();
+    if (grp == 1)
+        bar(); // the second group runs one slot behind
+    clear();
+
+    // One stage.  kSteady: every fetch below exists (the loop's body then has
+    // no branch but the tile switch: scalar work between the barriers costs
+    // MFMA time); else g is one of the last kSlots stages.
+    auto stage = [&](auto steady, int g) __attribute__((always_inline)) {
+        constexpr bool kSteady = decltype(steady)::value;
+        const int rem = stages - 1 - g; // stages after this one
+        if constexpr (kFour)
+        {
+            // phase 0: W0 X0; X1(g) next
+            read_w(0);
+            read_x(0);
+            if (kSteady || rem >= 1)
+                wait_vm<10>();
+            else
+                wait_vm<2>();
+            wait_lds();
+            bar();
+            mma(0, 0);
+            bar();
+            // phase 1: W0 X1; W0 X0 of stage g + 2; W1(g) next
+            read_x(1);
+            if constexpr (kSteady)
+            {
+                fetch_w(0);
+                fetch_x(0);
+                wait_vm<12>();
+            }
+            else if (rem >= 1)
+                wait_vm<8>();
+            else
+                wait_vm<0>();
+            wait_lds();
+            bar();
+            mma(0, 1);
+            bar();
+            // phase 2: W1 X1; X1 of stage g + 2
+            read_w(1);
+            if constexpr (kSteady)
+                fetch_x(1);
+            wait_lds();
+            bar();
+            mma(1, 1);
+            bar();
+            // phase 3: W1 X0; W1 of stage g + 2; W0 X0 of stage g + 1 next
+            if constexpr (kSteady)
+            {
+                fetch_w(1);
+                fetch_next();
+                wait_vm<12>();
+            }
+            else
+                wait_vm<4>();
+            bar();
+            mma(1, 0);
+            bar();
+        }
+        else if constexpr (MH + NH == 3)
+        {
+            // phase 0: W0 X0; the rest of stage g - 1 + kSlots; X1 / W1 of this stage next
+            read_w(0);
+            read_x(0);
+            if (g > 0 && (kSteady || rem >= kSlots - 1))
+            {
+                if constexpr (MH == 2)
+                    fetch_x(1);
+                else
+                    fetch_w(1);
+                fetch_next();
+            }
+            if constexpr (kSteady)
+                wait_vm<(kSlots - 1) * 6>();
+            else
+                wait_younger(min(rem, kSlots - 1) * 6);
+            wait_lds();
+            bar();
+            mma(0, 0);
+            bar();
+            // phase 1: X1 or W1; W0 X0 of stage g + kSlots; W0 X0 of stage g + 1 next
+            if constexpr (MH == 2)
+                read_x(1);
+            else
+                read_w(1);
+            if constexpr (kSteady)
+            {
+                fetch_w(0);
+                fetch_x(0);
+                wait_vm<2 + 6 * (kSlots - 2) + 4>();
+            }
+            else if (rem >= 2)
+                wait_younger(2 + 6 * (rem - 1));
+            else
+                wait_vm<2>();
+            wait_lds();
+            bar();
+            if constexpr (MH == 2)
+                mma(0, 1);
+            else
+                mma(1, 0);
+            bar();
+        }
+        else
+        {
+            read_w(0);
+            read_x(0);
+            if (g > 0 && (kSteady || rem >= kSlots - 1))
+            {
+                fetch_w(0);
+                fetch_x(0);
+                fetch_next();
+            }
+            if constexpr (kSteady)
+                wait_vm<(kSlots - 2) * 4>();
+            else
+                wait_younger(max(0, min(rem, kSlots - 1) - 1) * 4);
+            wait_lds();
+            bar();
+            mma(0, 0);
+            bar();
+        }
+        read_slot_next();
+    };
+    int g = 0;
+    for (int tile = 0; tile < ntiles; tile++)
+    {
+        const int steady = min(max(stages - kSlots - g, 0), nk);
+        int m0, n0;
+        tile_of(tile, &m0, &n0);
+        int i = 0;
+        if constexpr (EPI == kGemmResidual)
+        {
+            // the tile's residual lines move into the L2 while its last stages run
+#pragma nounroll
+            for (; i < steady - kTouchAhead; i++)
+                stage(std::true_type{}, g++);
+            // lane: line lane & (lines - 1) of row lane / lines of the wave's rows
+            constexpr int kLines = 2 * NH;            // 128-byte lines of a tile row
+            constexpr int kPerTouch = 64 / kLines;    // rows per instruction
+            constexpr int kRows = kHalf * MH / 8;     // rows of this wave
+#pragma unroll
+            for (int u = 0; u < kRows / kPerTouch; u++)
+            {
+                const int row = min(m0 + kRows * wave + kPerTouch * u + lane / kLines, a.m - 1);
+                touch(a.r + static_cast<long long>(row) * a.n + n0 + 64 * (lane % kLines),
+                      lds0 + kSlots * S::kStageBytes + wave * kEpiWave);
+            }
+        }
+#pragma nounroll
+        for (; i < steady; i++)
+            stage(std::true_type{}, g++);
+#pragma nounroll
+        for (; i < nk; i++)
+            stage(std::false_type{}, g++);
+        char* mine = smem + kSlots * S::kStageBytes + wave * kEpiWave;
+        if constexpr (KS)
+        {
+            // one tile per workgroup: the stage slots are free once both
+            // groups are done.  Each wave hands half of its sums to the wave
+            // that holds the same part for the other k-steps, and finishes
+            // the other half: group 0 X tiles 0, 1, group 1 X tiles 2, 3
+            if (grp == 0)
+                bar();
+            f4* give = reinterpret_cast<f4*>(smem) + wave * 8 * 64 + lane;
+            const f4* take = reinterpret_cast<const f4*>(smem) + (wave ^ 4) * 8 * 64 + lane;
+            f4 sum[1][1][4][2];
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int b = 0; b < 2; b++)
+                {
+                    give[(2 * t + b) * 64] = grp == 0 ? acc[0][0][t][2 + b] : acc[0][0][t][b];
+                    sum[0][0][t][b] = grp == 0 ? acc[0][0][t][b] : acc[0][0][t][2 + b];
+                }
+            wait_lds();
+            bar();
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int b = 0; b < 2; b++)
+                    sum[0][0][t][b] += take[(2 * t + b) * 64];
+            epilogue<1, 1, EPI>(a, sum, mine, m0 + xrow + 32 * grp, n0 + wrow, lane);
+            return;
+        }
+        else
+        {
+            epilogue<MH, NH, EPI>(a, acc, mine, m0 + xrow, n0 + wrow, lane);
+            clear();
+        }
+    }
+    if (grp == 0)
+        bar();
+}
+
+template <int MH, int NH, int EPI, bool KS = false>
+int launch(const TileArgs& a, hipStream_t stream)
+{
+    using S = Shape<MH, NH>;
+    const void* fn = reinterpret_cast<const void*>(&gemm_tile_kernel<MH, NH, EPI, KS>);
+    const int rc = set_dynamic_lds(fn, S::kLds, "gemm_f16: dynamic LDS attribute");
+    if (rc != SV2_OK)
+        return rc;
+    // a multiple of the 8 XCDs; KS: one tile per workgroup
+    const int all = (a.total + 7) / 8 * 8;
+    const int grid = KS ? all : std::min(kCus, all);
+    hipLaunchKernelGGL((gemm_tile_kernel<MH, NH, EPI, KS>), dim3(static_cast<unsigned>(grid)), dim3(kThreads), S::kLds,
+                       stream, a);
+    const hipError_t err = hipGetLastError();
+    return err == hipSuccess ? SV2_OK : hip_error(err, "gemm_tile_kernel launch");
+}
+
+// The tile forms and their measured times (us, MI355X, random operands): a
+// stage of 64 k of one tile when few CUs run (bounded by LDS) and when all of
+// them do (by power and the L2), and a tile's epilogue.
+enum Form
+{
+    kBig,   // 256 x 256
+    kTall,  // 256 rows x 128 columns
+    kSmall, // 128 x 128
+    kSplit, // 128 x 128, K split between the groups
+    kWide,  // SwiGLU: 128 rows x (128 gate + 128 value)
+    kForms
+};
+struct FormCost
+{
+    int rows, cols; // of W rows: SwiGLU outputs are half as many
+    double stage_min, stage_full, tile;
+};
+constexpr FormCost kCost[kForms] = {
+    {256, 256, 0.97, 1.42, 3.0}, {256, 128, 0.58, 0.78, 2.0}, {128, 128, 0.39, 0.50, 1.5},
+    {128, 128, 0.33, 0.42, 2.0}, {128, 256, 0.60, 0.80, 2.0},
+};
+constexpr double kLaunch = 7.0; // launch, first fetches, drain
+
+long long tiles_of(Form f, int rows, long long wrows)
+{
+    return (static_cast<long long>(rows) + kCost[f].rows - 1) / kCost[f].rows * (wrows / kCost[f].cols);
+}
+
+double form_us(Form f, int rows, int in, long long wrows)
+{
+    const long long tiles = tiles_of(f, rows, wrows);
+    const double nk = in / kBK;
+    const FormCost& c = kCost[f];
+    double us = kLaunch + static_cast<double>(tiles / kCus) * (nk * c.stage_full + c.tile);
+    const long long left = tiles % kCus;
+    if (left > 0)
+        us += nk * std::max(c.stage_min, c.stage_full * static_cast<double>(left) / kCus) + c.tile;
+    return us;
+}
+
+// How the rows of a product are tiled: all of them in one form, or, where the
+// last round of 256 x 256 tiles would leave most CUs idle, the row bands that
+// fill whole rounds in 256 x 256 tiles and the rest in another form (out
+// 6912 -> 2560 at 21658 rows is 3.3 rounds).  The choice depends on the sizes
+// alone.
+struct Plan
+{
+    Form first, rest;
+    int first_rows; // 0: all rows in `rest`
+    double us;
+};
+
+Plan make_plan(int rows, int in, int out, int epi, bool rounded)
+{
+    const long long wrows = epi == kGemmSwiGLU ? 2LL * out : out;
+    Form forms[4];
+    int nf = 0;
+    if (epi == kGemmSwiGLU)
+    {
+        forms[nf++] = kBig;
+        forms[nf++] = kWide;
+    }
+    else
+    {
+        if (out % 256 == 0)
+            forms[nf++] = kBig;
+        forms[nf++] = kTall;
+        forms[nf++] = kSmall;
+        // the rounded epilogues keep one order of summation in every form
+        if (!rounded)
+            forms[nf++] = kSplit;
+    }
+    Plan best{kBig, forms[0], 0, form_us(forms[0], rows, in, wrows)};
+    for (int i = 1; i < nf; i++)
+    {
+        const double us = form_us(forms[i], rows, in, wrows);
+        if (us < best.us)
+            best = Plan{kBig, forms[i], 0, us};
+    }
+    if (forms[0] != kBig)
+        return best;
+    const long long per_band = wrows / 256;
+    const long long bands = static_cast<long long>(kCus) * (tiles_of(kBig, rows, wrows) / kCus) / per_band;
+    const long long first = bands * 256;
+    if (first > 0 && first < rows)
+        for (int i = 1; i < nf; i++)
+        {
+            const double us = form_us(kBig, static_cast<int>(first), in, wrows) +
+                              form_us(forms[i], rows - static_cast<int>(first), in, wrows);
+            if (us < best.us)
+                best = Plan{kBig, forms[i], static_cast<int>(first), us};
+        }
+    return best;
+}
+
+template <int EPI>
+int launch_form(Form f, const TileArgs& a, hipStream_t stream)
+{
+    if constexpr (EPI == kGemmSwiGLU)
+    {
+        return f == kBig ? launch<2, 2, EPI>(a, stream) : launch<1, 2, EPI>(a, stream);
+    }
+    else
+    {
+        switch (f)
+        {
+        case kBig: return launch<2, 2, EPI>(a, stream);
+        case kTall: return launch<2, 1, EPI>(a, stream);
+        case kSmall: return launch<1, 1, EPI>(a, stream);
+        default: return launch<1, 1, EPI, true>(a, stream);
+        }
     }
 }
+
+// Rows r0 .. r0 + rows of the product in form f.
+int run_rows(Form f, TileArgs a, int epi, int r0, int rows, hipStream_t stream)
+{
+    const long long wrows = epi == kGemmSwiGLU ? 2LL * a.n : a.n;
+    a.x += static_cast<long long>(r0) * a.k;
+    a.y += static_cast<long long>(r0) * a.n;
+    if (a.r)
+        a.r += static_cast<long long>(r0) * a.n;
+    a.m = rows;
+    a.tiles_m = (rows + kCost[f].rows - 1) / kCost[f].rows;
+    a.tiles_n = static_cast<int>(wrows / kCost[f].cols);
+    const long long total = tiles_of(f, rows, wrows);
+    if (total > INT_MAX - kCus)
+        return set_error(SV2_EUNSUPPORTED, "inner product: too many tiles");
+    a.total = static_cast<int>(total);
+    // eight row bands a group: an XCD's 32 tiles are then 8 bands x 4 columns
+    a.group_m = 8;
+    switch (epi)
+    {
+    case kGemmStore: return launch_form<kGemmStore>(f, a, stream);
+    case kGemmResidual: return launch_form<kGemmResidual>(f, a, stream);
+    default: return launch_form<kGemmSwiGLU>(f, a, stream);
+    }
+}
+
+bool operands_fit(int rows, int in, int out)
+{
+    return static_cast<long long>(rows) * in * 2 <= INT_MAX && static_cast<long long>(out) * in * 2 <= INT_MAX;
+}
+
 } // namespace
 
 bool gemm_mfma_supported(int in, int out, int epi)
 {
     if (in <= 0 || in % kBK != 0 || out <= 0)
         return false;
-    return epi == kSwiGLU ? out % 128 == 0 : out % kBN == 0;
+    return epi == kGemmSwiGLU ? out % 128 == 0 : out % 256 == 0;
+}
+
+bool gemm_mfma_preferred(int rows, int in, int out, int epi, const void* x, const void* w, const void* w2,
+                         const void* y, const void* residual)
+{
+    // fewer rows leave most CUs without a tile; there the library's smaller
+    // tiles are as fast (96 rows, 6912 -> 2560: 22 us against 48)
+    return rows >= kPreferRows && gemm_mfma_supported(in, out, epi) && operands_fit(rows, in, out) &&
+           !misaligned(x, 16) && !misaligned(w, 16) && !misaligned(w2, 16) && !misaligned(y, 16) &&
+           !misaligned(residual, 16);
 }
 
 int gemm_mfma(hipStream_t stream, int rows, int in, int out, const void* x, const void* w, const void* w2, void* y,
-              int epi, const float* bias, const float* gate, const void* residual)
+              int epi, bool rounded, const float* bias, const float* gate, const void* residual)
 {
     if (rows == 0)
         return SV2_OK;
-    if (epi != kStore && epi != kResidual && epi != kSwiGLU)
+    if (epi != kGemmStore && epi != kGemmResidual && epi != kGemmSwiGLU)
         return set_error(SV2_EINVAL, "inner product: unknown epilogue");
     if (rows < 0 || !gemm_mfma_supported(in, out, epi))
         return set_error(SV2_EUNSUPPORTED,
                          "inner product: needs in a multiple of 64 and out a multiple of 256 (SwiGLU: 128)");
-    if (!x || !w || !y || (epi == kResidual && !residual) || (epi == kSwiGLU && !w2))
+    if (!x || !w || !y || (epi == kGemmResidual && !residual) || (epi == kGemmSwiGLU && !w2))
         return set_error(SV2_EINVAL, "inner product: null pointer");
     if (misaligned(x, 16) || misaligned(w, 16) || misaligned(w2, 16) || misaligned(y, 16) || misaligned(residual, 16))
         return set_error(SV2_EINVAL, "inner product: x, W, y and residual must be 16-byte aligned");
-    // the operands are read through buffer resources with 32-bit byte offsets
-    // (the kernel forms them unsigned, so padded tile rows past `rows` stay
-    // exact; see make_operands)
-    if (static_cast<long long>(rows) * in * 2 > INT_MAX || static_cast<long long>(out) * in * 2 > INT_MAX)
+    if (!operands_fit(rows, in, out))
         return set_error(SV2_EUNSUPPORTED, "inner product: an operand exceeds 2 GiB");
-    const int rc = set_dynamic_lds(reinterpret_cast<const void*>(&gemm_f16_kernel), kLds,
-                                   "gemm_mfma: dynamic LDS attribute");
-    if (rc != SV2_OK)
-        return rc;
-    GemmArgs a;
+    TileArgs a{};
     a.x = static_cast<const _Float16*>(x);
     a.w = static_cast<const _Float16*>(w);
     a.w2 = static_cast<const _Float16*>(w2);
     a.y = static_cast<_Float16*>(y);
-    a.r = static_cast<const _Float16*>(residual);
+    a.r = static_cast<const _Float16*>(epi == kGemmResidual ? residual : nullptr);
     a.bias = bias;
     a.gate = gate;
-    a.m = rows;
     a.n = out;
     a.k = in;
-    a.epi = epi;
-    a.tiles_n = epi == kSwiGLU ? out / 128 : out / kBN;
-    const long long tiles = static_cast<long long>((rows + kBM - 1) / kBM) * a.tiles_n;
-    if (tiles >= (1LL << 31))
-        return set_error(SV2_EUNSUPPORTED, "gemm_mfma: too many tiles");
-    hipLaunchKernelGGL(gemm_f16_kernel, dim3(static_cast<unsigned>(tiles)), dim3(kThreads), kLds, stream, a);
-    const hipError_t err = hipGetLastError();
-    return err == hipSuccess ? SV2_OK : hip_error(err, "gemm_f16_kernel launch");
+    a.rounded = rounded ? 1 : 0;
+    const Plan plan = make_plan(rows, in, out, epi, rounded);
+    if (plan.first_rows > 0)
+    {
+        const int rc = run_rows(plan.first, a, epi, 0, plan.first_rows, stream);
+        if (rc != SV2_OK)
+            return rc;
+    }
+    return run_rows(plan.rest, a, epi, plan.first_rows, rows - plan.first_rows, stream);
 }
 
 } // namespace sv2
@@ -492,7 +942,7 @@ try
                   "epilogue codes of the C ABI and the kernel agree");
     if (epilogue != SV2_EPI_SWIGLU && w_value)
         return sv2::set_error(SV2_EINVAL, "sv2_inner_product_f16: w_value is only read by SV2_EPI_SWIGLU");
-    return sv2::gemm_mfma(static_cast<hipStream_t>(stream), rows, in, out, x, w, w_value, y, epilogue, bias, gate,
+    return sv2::gemm_mfma(static_cast<hipStream_t>(stream), rows, in, out, x, w, w_value, y, epilogue, true, bias, gate,
                           residual);
 }
 catch (...)

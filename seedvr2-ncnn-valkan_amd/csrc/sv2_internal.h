@@ -158,9 +158,8 @@ int launch_residual_table(void* x, const void* residual, int dtype, int rows, in
 
 // y[rows, out] = x[rows, in] W^T, W [out][in] row-major (an InnerProduct
 // without its bias), in dtype (SV2_F32 or SV2_F16); enqueued on `stream`.
-// fp16 runs on hipBLASLt with fp32 accumulation (the first product of a
-// shape times the library's candidate kernels and synchronises the stream
-// once); fp32 on gemm_f32_exact.
+// fp16 runs with fp32 accumulation on gemm_mfma where gemm_mfma_preferred says
+// so, else on hipBLASLt; fp32 on gemm_f32_exact.
 int gemm_rows(hipStream_t stream, int dtype, int rows, int in, int out, const void* x, const void* w, void* y);
 // The same with the InnerProduct's bias (may be NULL): fp32 adds it to the
 // double sum before the one rounding; fp16 adds it in a pass after the product.
@@ -172,22 +171,28 @@ int gemm_f32_exact(hipStream_t stream, int rows, int in, int out, const float* x
                    float* y);
 // fp16 only: y = gate[c] * (x W^T)[r][c] + residual[r][c] (+ bias[c] when
 // bias is not null), the gated residual of seedvr2_dit_block.cpp:807-825 in
-// the product's epilogue (fp32, one rounding to fp16); -2 when hipBLASLt has
-// no kernel for it.  A preceding InnerProduct bias b enters as bias = gate * b.
+// the product's epilogue (fp32, one rounding to fp16), on gemm_mfma or
+// hipBLASLt as gemm_rows; -2 when hipBLASLt has no kernel for it.  A preceding InnerProduct bias b enters as bias = gate * b.
 int gemm_rows_gated(hipStream_t stream, int dtype, int rows, int in, int out, const void* x, const void* w, void* y,
                     const float* gate, const void* residual, const float* bias = nullptr);
 
 // fp16 y = epilogue(x W^T) on the hand-written MFMA kernel (gemm.hip), x
-// [rows][in], W (and w2) [out][in].  Epilogues: store; the gated residual
-// y = fp16((fp16(x W^T) + bias) * gate + residual) (bias, gate optional);
-// SwiGLU y = silu(fp16(x W^T)) * fp16(x W2^T).  Needs in % 64 == 0 and
-// out % 256 == 0 (SwiGLU: out % 128 == 0).
+// [rows][in], W (and w2) [out][in].  Epilogues, in fp32 with one rounding:
+// store; the gated residual y = fp16(x W^T * gate + residual + bias) (bias,
+// gate optional); SwiGLU y = fp16(silu(x W^T) * x W2^T).  `rounded`: the
+// products are rounded to fp16 first and the bias is added before the gate,
+// y = fp16((fp16(x W^T) + bias) * gate + residual).  Needs in % 64 == 0 and
+// out % 256 == 0 (SwiGLU: out % 128 == 0), operands of at most 2 GiB and
+// 16-byte aligned x, W, y and residual.
 constexpr int kGemmStore = 0;
 constexpr int kGemmResidual = 1;
 constexpr int kGemmSwiGLU = 2;
 bool gemm_mfma_supported(int in, int out, int epi);
+// Whether the fp16 products of gemm_rows and its kin take that kernel.
+bool gemm_mfma_preferred(int rows, int in, int out, int epi, const void* x, const void* w, const void* w2,
+                         const void* y, const void* residual);
 int gemm_mfma(hipStream_t stream, int rows, int in, int out, const void* x, const void* w, const void* w2, void* y,
-              int epi, const float* bias, const float* gate, const void* residual);
+              int epi, bool rounded, const float* bias, const float* gate, const void* residual);
 
 // fp16 y = epilogue(x W^T) for 1-64 rows on the weight-streaming kernel
 // (gemm_few.hip), the same epilogues as gemm_mfma (kGemmStore also takes an

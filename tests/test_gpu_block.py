@@ -604,3 +604,24 @@ def test_rows_not_merged_for_last_layer_or_captures(hip, device):
             assert blk.last_forward_merged() == (not last and not capture), (last, capture)
         finally:
             blk.close()
+
+
+@pytest.mark.parametrize("grid,L", [((1, 15, 17), 1), ((1, 16, 16), 64), ((2, 16, 30), 58),
+                                    ((3, 20, 23), 65), ((5, 24, 24), 2)])
+def test_fp16_products_around_the_kernel_choice(hip, orc, device, grid, L):
+    """fp16 block on either side of the row count where its products move to
+    the MFMA kernel (255 and 256 video rows), with a ragged last tile band, and
+    with up to 2880 rows, against the oracle."""
+    T, H, W = grid
+    dim, heads, hidden = 256, 2, 512
+    print(f"[kernel choice] grid={grid} L={L}", flush=True)
+    rng = np.random.default_rng(T * H * W + L)
+    w = nf.random_weights(rng, dim, hidden, shared=True)
+    rows = rng.standard_normal((T * H * W + L, dim), dtype=np.float32).astype(np.float16).astype(np.float32)
+    emb = rng.standard_normal(6 * dim, dtype=np.float32)
+    cfg = hip.block_config(dim=dim, heads=heads, mlp_hidden=hidden, shared_weights=1, shifted_window=1, block_index=10)
+    blk = hip.DitBlock.from_host(cfg, w, hip.F16)
+    try:
+        compare(hip, orc, blk, w, rows[:T * H * W], rows[T * H * W:], emb, T, H, W, device, f"choice {grid} {L}")
+    finally:
+        blk.close()

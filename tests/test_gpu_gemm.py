@@ -86,6 +86,31 @@ def test_store(hip, rows, k, n):
     assert mean < 2e-4
 
 
+@pytest.mark.parametrize("rows,k,n", [
+    (1, 64, 256),        # one stage, one row of a tile
+    (128, 128, 512),     # two stages, fewer than any ring holds
+    (129, 192, 256),     # three stages, one row in the second tile
+    (700, 2560, 2560),   # 128 x 128 tiles
+    (960, 2560, 7680),   # 256 x 128 tiles
+    (2049, 1280, 7680),  # 256 x 256 tiles in one round, one row in the last band
+    (6700, 640, 2560),   # 256 x 256 tiles over one round, the last one short
+    (7300, 320, 7680),   # whole rounds of 256 x 256 tiles and a rest in another form
+])
+def test_store_tile_forms(hip, rows, k, n):
+    """The tile forms and the edges of their ranges; rows past the output stay untouched."""
+    print(f"[tile form] rows={rows} in={k} out={n}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(rows * 3 + k + n)
+    x = rand16((rows, k), 1.0, gen)
+    w = rand16((n, k), 0.02, gen)
+    y = torch.full((rows + 2, n), 7.0, dtype=torch.float16, device="cuda")
+    hip.inner_product_f16(x, w, y[:rows])
+    torch.cuda.synchronize()
+    assert bool((y[rows:] == 7.0).all())
+    idx = sample_rows(rows)
+    ref, slack = reference64(x, w, idx)
+    assert_ulp(y[:rows].cpu().numpy()[idx], ref, slack=slack)
+
+
 @pytest.mark.parametrize("rows", [21600, 777])
 @pytest.mark.parametrize("bias,gate", [(True, True), (False, True), (True, False)])
 def test_residual(hip, rows, bias, gate):
