@@ -2,11 +2,11 @@
 //
 // fp16 (the fast mode), fp32 accumulation: gemm_mfma (gemm.hip) where
 // gemm_mfma_preferred says so, by the sizes and alignments alone; else
-// hipBLASLt.  The first library product of a shape on a device plans it: the library's best-ranked kernel that needs
-// no workspace, kept for the rest of the process.  The choice depends on the
-// shape alone, so a shape is computed with the same kernel (and rounds the
-// same way) in every process, and planning neither runs nor synchronises
-// anything.  (Timing the library's 16 best-ranked kernels instead and keeping
+// hipBLASLt.  The first library product of a shape on a device plans it: the
+// library's best-ranked kernel that needs no workspace, kept for the rest of
+// the process.  The choice depends on the shape alone, so a shape is computed
+// with the same kernel (and rounds the same way) in every process, and
+// planning neither runs nor synchronises anything.  (Timing the library's 16 best-ranked kernels instead and keeping
 // the fastest changed the 720p DiT step by less than its run-to-run spread.)
 // Without a workspace, products on different streams share nothing.  The
 // gated form carries the block's gated residual in the library's epilogue
@@ -241,7 +241,11 @@ int gemm_rows_gated(hipStream_t stream, int dtype, int rows, int in, int out, co
     if (gemm_mfma_preferred(rows, in, out, kGemmResidual, x, w, nullptr, y, residual))
         return gemm_mfma(stream, rows, in, out, x, w, nullptr, y, kGemmResidual, false, bias, gate, residual);
     const Gated g{gate, residual, bias};
-    return gemm_f16(stream, rows, in, out, x, w, y, &g);
+    const int rc = gemm_f16(stream, rows, in, out, x, w, y, &g);
+    // sizes the library has no kernel without a workspace for
+    if (rc == SV2_EUNSUPPORTED && gemm_mfma_fits(rows, in, out, kGemmResidual, x, w, nullptr, y, residual))
+        return gemm_mfma(stream, rows, in, out, x, w, nullptr, y, kGemmResidual, false, bias, gate, residual);
+    return rc;
 }
 
 int gemm_rows(hipStream_t stream, int dtype, int rows, int in, int out, const void* x, const void* w, void* y)

@@ -33,9 +33,9 @@
 //
 // What bounds it, 21658 rows (MI355X; the library product beside it):
 //   qkv 2560 -> 7680                   594 us (1.43 PFLOP/s)   589
-//   proj 2560 -> 2560 + residual       250 us                  276 (its residual apart)
+//   proj 2560 -> 2560 + residual       250 us                  276
 //   gate/in 2560 -> 2 x 6912 + SwiGLU  1062 us                 1067 + 137
-//   out 6912 -> 2560 + residual        605 us                  676 (its residual apart)
+//   out 6912 -> 2560 + residual        605 us                  676
 // With all-zero operands the same launches take 434 / 215 / 773 / 512 us: on
 // random data the clock drops under the matrix cores' power, and the rest is
 // LDS bandwidth (192 KB of operand reads and 64 KB of fetch a 256 x 256 stage,
@@ -749,7 +749,7 @@ struct FormCost
 };
 constexpr FormCost kCost[kForms] = {
     {256, 256, 0.97, 1.42, 3.0}, {256, 128, 0.58, 0.78, 2.0}, {128, 128, 0.39, 0.50, 1.5},
-    {128, 128, 0.33, 0.42, 2.0}, {128, 256, 0.60, 0.80, 2.0},
+    {128, 128, 0.33, 0.48, 2.0}, {128, 256, 0.60, 0.80, 2.0},
 };
 constexpr double kLaunch = 7.0; // launch, first fetches, drain
 
@@ -874,6 +874,27 @@ bool operands_fit(int rows, int in, int out)
     return static_cast<long long>(rows) * in * 2 <= INT_MAX && static_cast<long long>(out) * in * 2 <= INT_MAX;
 }
 
+// Whether a residual product is faster here than the library's product with
+// the residual in its epilogue.  Its 2560 columns make a third of qkv's tiles,
+// so most sizes leave CUs idle in the only or the last round, where the
+// library's tiles (192 x 256, 256 x 64 and others) divide better.  Inside a
+// block, out 6912 -> 2560 and proj 2560 -> 2560, library against this kernel:
+//   1018 rows   out 46 us / 61, proj 22 / 22      2065   78 / 97, 38 / 38
+//   4273        out 123 / 139, proj 60 / 68       10849  284 / 301, 124 / 139
+// This kernel wins where one round of `kSplit` tiles fills the CUs and K is
+// short (proj at 1361 rows 29 us / 22; at K = 6912 both take 60), and from two
+// whole 256 x 256 rounds with the third no less than a quarter full (17329
+// rows: out 506 / 472, proj 227 / 224; but 19489 rows, 3.01 rounds: 509 / 536,
+// 209 / 247).
+bool residual_pays(int rows, int in, int out)
+{
+    const long long split = tiles_of(kSplit, rows, out);
+    if (in <= out && split <= kCus && 10 * split >= 7 * kCus)
+        return true;
+    const long long big = tiles_of(kBig, rows, out);
+    return big / kCus >= 2 && 4 * (big % kCus) >= kCus;
+}
+
 } // namespace
 
 bool gemm_mfma_supported(int in, int out, int epi)
@@ -883,14 +904,20 @@ bool gemm_mfma_supported(int in, int out, int epi)
     return epi == kGemmSwiGLU ? out % 128 == 0 : out % 256 == 0;
 }
 
+bool gemm_mfma_fits(int rows, int in, int out, int epi, const void* x, const void* w, const void* w2, const void* y,
+                    const void* residual)
+{
+    return rows > 0 && gemm_mfma_supported(in, out, epi) && operands_fit(rows, in, out) && !misaligned(x, 16) &&
+           !misaligned(w, 16) && !misaligned(w2, 16) && !misaligned(y, 16) && !misaligned(residual, 16);
+}
+
 bool gemm_mfma_preferred(int rows, int in, int out, int epi, const void* x, const void* w, const void* w2,
                          const void* y, const void* residual)
 {
     // fewer rows leave most CUs without a tile; there the library's smaller
     // tiles are as fast (96 rows, 6912 -> 2560: 22 us against 48)
-    return rows >= kPreferRows && gemm_mfma_supported(in, out, epi) && operands_fit(rows, in, out) &&
-           !misaligned(x, 16) && !misaligned(w, 16) && !misaligned(w2, 16) && !misaligned(y, 16) &&
-           !misaligned(residual, 16);
+    return rows >= kPreferRows && gemm_mfma_fits(rows, in, out, epi, x, w, w2, y, residual) &&
+           (epi != kGemmResidual || residual_pays(rows, in, out));
 }
 
 int gemm_mfma(hipStream_t stream, int rows, int in, int out, const void* x, const void* w, const void* w2, void* y,

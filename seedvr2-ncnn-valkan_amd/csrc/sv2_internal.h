@@ -188,6 +188,9 @@ constexpr int kGemmStore = 0;
 constexpr int kGemmResidual = 1;
 constexpr int kGemmSwiGLU = 2;
 bool gemm_mfma_supported(int in, int out, int epi);
+// Whether that kernel takes these operands at all.
+bool gemm_mfma_fits(int rows, int in, int out, int epi, const void* x, const void* w, const void* w2, const void* y,
+                    const void* residual);
 // Whether the fp16 products of gemm_rows and its kin take that kernel.
 bool gemm_mfma_preferred(int rows, int in, int out, int epi, const void* x, const void* w, const void* w2,
                          const void* y, const void* residual);

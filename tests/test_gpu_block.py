@@ -625,3 +625,21 @@ def test_fp16_products_around_the_kernel_choice(hip, orc, device, grid, L):
         compare(hip, orc, blk, w, rows[:T * H * W], rows[T * H * W:], emb, T, H, W, device, f"choice {grid} {L}")
     finally:
         blk.close()
+
+
+def test_fp16_residual_products_on_split_tiles(hip, orc, device):
+    """5768 rows at width 512: the residual products take one round of 128 x 128
+    tiles with K split between the wave groups (184 tiles, a ragged last band);
+    against the oracle."""
+    T, H, W, L = 6, 31, 31, 2
+    dim, heads, hidden = 512, 4, 512
+    rng = np.random.default_rng(5768)
+    w = nf.random_weights(rng, dim, hidden, shared=True)
+    rows = rng.standard_normal((T * H * W + L, dim), dtype=np.float32).astype(np.float16).astype(np.float32)
+    emb = rng.standard_normal(6 * dim, dtype=np.float32)
+    cfg = hip.block_config(dim=dim, heads=heads, mlp_hidden=hidden, shared_weights=1, shifted_window=1, block_index=10)
+    blk = hip.DitBlock.from_host(cfg, w, hip.F16)
+    try:
+        compare(hip, orc, blk, w, rows[:T * H * W], rows[T * H * W:], emb, T, H, W, device, "split tiles")
+    finally:
+        blk.close()
