@@ -324,26 +324,35 @@ struct BlockAda
     int tables;
 };
 
-__global__ __launch_bounds__(256) void block_tables_kernel(const float* emb, BlockAda a, int dim, float* out)
+// Latency alone: one table a block row, every load of a thread in flight at
+// once (the tables one after the other in each thread, whose stores keep the
+// next table's loads behind them: 5.8 us against 4.5 at dim 2560).
+__global__ __launch_bounds__(256) void block_tables_kernel(const float* __restrict__ emb, BlockAda a, int dim,
+                                                           float* __restrict__ out)
 {
 #pragma clang fp contract(off)
     const int c = blockIdx.x * 256 + threadIdx.x;
+    const int t = blockIdx.y;
     if (c >= dim)
         return;
-    for (int t = 0; t < a.tables; t++)
-    {
-        const int slot = (t & 1) ? 3 : 0;
-        float* o = out + static_cast<long long>(3 * t) * dim;
-        o[c] = emb[c * 6 + slot + 1] + a.scale[t][c];
-        o[dim + c] = emb[c * 6 + slot];
-        if (a.gate[t])
-            o[2 * dim + c] = emb[c * 6 + slot + 2] + a.gate[t][c];
-    }
-    if (a.bias)
+    if (t == a.tables) // the gated bias
     {
         const float g = emb[c * 6 + 2] + a.gate[0][c];
         out[12LL * dim + c] = g * a.bias[c];
+        return;
     }
+    const int slot = (t & 1) ? 3 : 0;
+    const float* gate = a.gate[t];
+    const float scale = a.scale[t][c];
+    const float gated = gate ? gate[c] : 0.f;
+    const float e0 = emb[c * 6 + slot];
+    const float e1 = emb[c * 6 + slot + 1];
+    const float e2 = emb[c * 6 + slot + 2];
+    float* o = out + static_cast<long long>(3 * t) * dim;
+    o[c] = e1 + scale;
+    o[dim + c] = e0;
+    if (gate)
+        o[2 * dim + c] = e2 + gated;
 }
 
 // silu(g) * v with silu(g) = g / (1 + exp(-g)) (seedvr2_dit_block.cpp:58-61, :1103-1109).
@@ -641,7 +650,8 @@ int launch_block_tables(const float* emb, const float* const* scale, const float
     }
     a.bias = bias;
     a.tables = tables;
-    hipLaunchKernelGGL(block_tables_kernel, dim3((dim + 255) / 256), dim3(256), 0, stream, emb, a, dim, out);
+    hipLaunchKernelGGL(block_tables_kernel, dim3((dim + 255) / 256, tables + (bias ? 1 : 0)), dim3(256), 0, stream, emb, a,
+                       dim, out);
     const hipError_t err = hipGetLastError();
     return err == hipSuccess ? SV2_OK : hip_error(err, "block_tables_kernel launch");
 }
