@@ -203,3 +203,10 @@ def test_stages_one_at_a_time_equal_the_combined_call(hip, device, dtype):
         torch.cuda.synchronize()
         assert torch.equal(ov, ref_v), split
         assert torch.equal(ot, ref_t), split
+
+
+@pytest.mark.parametrize("windows", [1, 15, 16, 17, 33])
+def test_text_average_over_window_counts(hip, orc, device, windows):
+    """Text rows averaged over counts of windows around the reduction's batches of 16."""
+    _case(hip, orc, device, T=1, H=3, W=4 * windows, Lt=5, heads=2, shifted=False, wt=1, wh=3, ww=4,
+          in_dtype="f16", out_dtype="f16", seed=windows)
