@@ -215,7 +215,14 @@ __device__ inline void wait_younger(int n)
 // time go through `mine` (2 KB of LDS, this wave's own), 16-byte chunk c of
 // row r in slot c ^ (r & 7), so that residual rows are read and output rows
 // written as whole 128-byte lines.
-template <int MH, int NH, int EPI>
+//
+// SwiGLU's silu: with `ROUNDED` expf and an IEEE divide, 2.5 fp32 ulps at most
+// in all; else exp2 and the reciprocal, as the separate 16-bit pass has them
+// (up to 8 ulps where the gate is large and negative: the fp32 rounding of the
+// exponent, below the fp16 roundings of g and u that this form leaves out).
+// Two bodies, not a branch per element: the first costs gate/in at 21658 rows
+// 1166 us where the second takes 1107.
+template <int MH, int NH, int EPI, bool ROUNDED>
 __device__ __forceinline__ void epilogue(const TileArgs& a, f4 (&acc)[NH][MH][4][2], char* mine, int row0, int col0, int lane)
 {
     constexpr bool kSw = EPI == kGemmSwiGLU;
@@ -288,18 +295,19 @@ __device__ __forceinline__ void epilogue(const TileArgs& a, f4 (&acc)[NH][MH][4]
                         float v = acc[h][j][t][b][e];
                         if constexpr (kSw)
                         {
-                            // silu(g) u: exp2 and the reciprocal, each within
-                            // an fp32 ulp, in place of expf and a divide (about
-                            // 45 instructions an element, 1197 us against 1074
-                            // for gate/in at 21658 rows)
                             float u = acc[NH - 1][j][t][b][e];
-                            if (a.rounded)
+                            if constexpr (ROUNDED)
                             {
                                 v = round16(v);
                                 u = round16(u);
+                                const float den = 1.f + expf(-v);
+                                v = (v / den) * u;
                             }
-                            const float den = 1.f + __builtin_amdgcn_exp2f(v * -kLog2e);
-                            v = v * __builtin_amdgcn_rcpf(den) * u;
+                            else
+                            {
+                                const float den = 1.f + __builtin_amdgcn_exp2f(v * -kLog2e);
+                                v = v * __builtin_amdgcn_rcpf(den) * u;
+                            }
                         }
                         if constexpr (EPI == kGemmResidual)
                         {
@@ -700,12 +708,15 @@ __global__ __launch_bounds__(kThreads) void gemm_tile_kernel(TileArgs a)
 #pragma unroll
                 for (int b = 0; b < 2; b++)
                     sum[0][0][t][b] += take[(2 * t + b) * 64];
-            epilogue<1, 1, EPI>(a, sum, mine, m0 + xrow + 32 * grp, n0 + wrow, lane);
+            epilogue<1, 1, EPI, false>(a, sum, mine, m0 + xrow + 32 * grp, n0 + wrow, lane);
             return;
         }
         else
         {
-            epilogue<MH, NH, EPI>(a, acc, mine, m0 + xrow, n0 + wrow, lane);
+            if (EPI == kGemmSwiGLU && a.rounded)
+                epilogue<MH, NH, EPI, true>(a, acc, mine, m0 + xrow, n0 + wrow, lane);
+            else
+                epilogue<MH, NH, EPI, false>(a, acc, mine, m0 + xrow, n0 + wrow, lane);
             clear();
         }
     }

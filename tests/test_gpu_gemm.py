@@ -154,6 +154,32 @@ def test_swiglu(hip, rows, k, f):
     assert_ulp(y.float().cpu().numpy(), ref)
 
 
+@pytest.mark.parametrize("rows", [64, 256])
+def test_swiglu_as_exact_as_expf_and_a_divide(hip, rows):
+    """silu(g) u of the entry point (`rounded` products) to fp32 accuracy: with
+    rows of the identity as X every product is one fp16 weight, so g and u are
+    known, and y is the fp16 rounding of a value within the error of expf (1
+    ulp), an addition, an IEEE divide and a multiplication (half an ulp each):
+    2.5 * 2^-23 of the float64 result.  Gates from -2 to -20, where an
+    exponent rounded to fp32 before an exp2 is off by several ulps.  64 rows
+    take one tile form, 256 the other; every row repeats the first 64."""
+    k, f = 64, 1 << 16
+    rng = np.random.default_rng(17)
+    g = (-rng.uniform(2.0, 20.0, (f, k))).astype(np.float16)
+    u = (2.0 ** rng.uniform(6.0, 12.0, (f, k))).astype(np.float16)
+    x = torch.eye(k, dtype=torch.float16, device="cuda").repeat(rows // k, 1).contiguous()
+    y = torch.empty((rows, f), dtype=torch.float16, device="cuda")
+    hip.inner_product_f16(x, torch.from_numpy(g).cuda(), y, hip.EPI_SWIGLU, w_value=torch.from_numpy(u).cuda())
+    torch.cuda.synchronize()
+    assert torch.equal(y, y[:k].repeat(rows // k, 1))
+    gd = g.T.astype(np.float64)
+    exact = gd / (1.0 + np.exp(-gd)) * u.T.astype(np.float64)
+    bound = 2.5 * 2.0 ** -23
+    low, high = (exact * (1 + bound)).astype(np.float16), (exact * (1 - bound)).astype(np.float16)
+    got = y[:k].cpu().numpy()
+    assert int(((got < low) | (got > high)).sum()) == 0
+
+
 def test_unsupported_shapes(hip):
     x = torch.zeros((4, 48), dtype=torch.float16, device="cuda")
     w = torch.zeros((256, 48), dtype=torch.float16, device="cuda")
