@@ -20,8 +20,11 @@ namespace
 {
 
 constexpr int kThreads = 256;
-constexpr int kReduceBlocks = 1024; // partial sums of the guidance statistics
-constexpr int kScaleBlocks = 256;   // blocks of the rescale, one per CU
+constexpr int kSumThreads = 1024;   // of the guidance with statistics and of the rescale
+constexpr int kReduceBlocks = 1024; // at most: partial sums of the guidance statistics
+constexpr int kScaleBlocks = 512;   // at most: blocks of the rescale, two per CU
+static_assert(kReduceBlocks <= kSumThreads, "a thread of the rescale takes one block's partials");
+static_assert(kSumThreads == 1024, "16 waves of four sums are one value a lane");
 
 unsigned blocks_for(long long n)
 {
@@ -115,70 +118,111 @@ __global__ __launch_bounds__(kThreads) void cfg_kernel(const float* pos, const f
         out[k] = guide(pos[k], neg[k], scale);
 }
 
-// With the rescale each block also writes its double sums of pos, pos^2, out,
-// out^2 (grid-stride over the elements, fixed order per block).
-__global__ __launch_bounds__(kThreads) void cfg_sums_kernel(const float* pos, const float* neg, float* out,
-                                                            long long count, float scale, double* partial)
+// Lane l of the wave gets the sum over its lanes of v[l % 4]: two halving
+// exchanges, then four of one value (a sum of each value by itself takes 24).
+__device__ inline double wave_sum4(const double (&v)[4], int lane)
 {
-    double sp = 0.0, spp = 0.0, so = 0.0, soo = 0.0;
-    const long long stride = static_cast<long long>(gridDim.x) * kThreads;
-    for (long long i = static_cast<long long>(blockIdx.x) * kThreads + threadIdx.x; i < count; i += stride)
-    {
-        const float p = pos[i];
-        const float o = guide(p, neg[i], scale);
-        out[i] = o;
-        sp += p;
-        spp += static_cast<double>(p) * p;
-        so += o;
-        soo += static_cast<double>(o) * o;
-    }
-    __shared__ double red[4][kThreads];
-    red[0][threadIdx.x] = sp;
-    red[1][threadIdx.x] = spp;
-    red[2][threadIdx.x] = so;
-    red[3][threadIdx.x] = soo;
+    const bool odd = lane & 1;
+    const bool high = lane & 2;
+    const double a = (odd ? v[1] : v[0]) + __shfl_xor(odd ? v[0] : v[1], 1);
+    const double b = (odd ? v[3] : v[2]) + __shfl_xor(odd ? v[2] : v[3], 1);
+    double s = (high ? b : a) + __shfl_xor(high ? a : b, 2);
+#pragma unroll
+    for (int d = 4; d < 64; d <<= 1)
+        s += __shfl_xor(s, d);
+    return s;
+}
+
+// The same over a block of kSumThreads, in every wave: 16 waves of 4 sums are
+// one value a lane.
+__device__ inline double block_sum4(const double (&v)[4], double* red)
+{
+    const int lane = threadIdx.x & 63;
+    const double s = wave_sum4(v, lane);
+    if (lane < 4)
+        red[4 * (threadIdx.x >> 6) + lane] = s;
     __syncthreads();
-    for (int s = kThreads / 2; s > 0; s >>= 1)
+    double t = red[lane];
+#pragma unroll
+    for (int d = 4; d < 64; d <<= 1)
+        t += __shfl_xor(t, d);
+    return t;
+}
+
+// With the rescale each block also writes its double sums of pos, pos^2, out,
+// out^2 (grid-stride over the quads, fixed order).  Blocks of 1024: a quad a
+// thread fills a CU and leaves few partials for the next kernel to add (338 at
+// the 720p clip, where blocks of 256 left the most there may be, 1024).
+__global__ __launch_bounds__(kSumThreads) void cfg_sums_kernel(const float* pos, const float* neg, float* out,
+                                                               long long count, float scale, double* partial)
+{
+    __shared__ double red[64];
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
+    auto add = [&](float p, float o) {
+        v[0] += p;
+        v[1] += static_cast<double>(p) * p;
+        v[2] += o;
+        v[3] += static_cast<double>(o) * o;
+    };
+    const long long stride = 4LL * gridDim.x * kSumThreads;
+    for (long long i = 4 * (static_cast<long long>(blockIdx.x) * kSumThreads + threadIdx.x); i < count; i += stride)
     {
-        if (static_cast<int>(threadIdx.x) < s)
-            for (int k = 0; k < 4; k++)
-                red[k][threadIdx.x] += red[k][threadIdx.x + s];
-        __syncthreads();
+        if (i + 4 <= count)
+        {
+            const f4 p = *reinterpret_cast<const f4*>(pos + i);
+            const f4 n = *reinterpret_cast<const f4*>(neg + i);
+            f4 o;
+            for (int e = 0; e < 4; e++)
+            {
+                o[e] = guide(p[e], n[e], scale);
+                add(p[e], o[e]);
+            }
+            *reinterpret_cast<f4*>(out + i) = o;
+            continue;
+        }
+        for (long long k = i; k < count; k++)
+        {
+            const float p = pos[k];
+            const float o = guide(p, neg[k], scale);
+            out[k] = o;
+            add(p, o);
+        }
     }
+    const double s = block_sum4(v, red);
     if (threadIdx.x < 4)
-        partial[blockIdx.x * 4 + threadIdx.x] = red[threadIdx.x][0];
+        partial[static_cast<long long>(blockIdx.x) * 4 + threadIdx.x] = s;
 }
 
 // sampler.cpp:41-62 (unbiased standard deviation from the sums) and :219-235:
 // factor = rescale * std(pos) / std(out) + (1 - rescale) when std(out) > 0,
-// then the outputs times it.  Every block forms the factor itself (a launch
-// of one block for it cost 2.8 us of the small clip's 13): thread t adds the
-// partials of blocks t, t + 256, ... in that order, then a fixed tree over the
-// threads, so the factor is the same in all of them and does not depend on
-// scheduling.  At most kScaleBlocks blocks, each reading the partials (32 KB
-// at most) once.
-__global__ __launch_bounds__(kThreads) void cfg_scale_kernel(const double* partial, int nblocks, float* out,
-                                                             long long count, float rescale)
+// then the outputs times it.  Every block forms the factor itself: thread t
+// takes the partials of block t (at most kReduceBlocks of them), the sums
+// follow in a fixed order, so the factor is the same in all blocks and does not
+// depend on scheduling.  A thread's first quad is requested before that.
+//
+// Bound by launch and the chain partials - sums - factor - product.  Guidance
+// and rescale together, in a graph: 9.8 us at the 720p clip, 6.0 at the
+// smallest.  With 256 blocks of 256 threads, each adding 1024 partials through
+// an eight-level tree of barriers before it streamed, 12.8 and 6.3; with 5400
+// blocks and a launch of its own for the factor, 11.7 and 7.3.
+__global__ __launch_bounds__(kSumThreads) void cfg_scale_kernel(const double* partial, int nblocks, float* out,
+                                                                long long count, float rescale)
 {
-    __shared__ double red[4][kThreads];
+    __shared__ double red[64];
     __shared__ float factor[2];
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int b = threadIdx.x; b < nblocks; b += kThreads)
+    const int tid = threadIdx.x;
+    long long i = 4 * (static_cast<long long>(blockIdx.x) * kSumThreads + tid);
+    f4 o = {0.f, 0.f, 0.f, 0.f};
+    if (i + 4 <= count)
+        o = *reinterpret_cast<const f4*>(out + i);
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
+    if (tid < nblocks)
         for (int k = 0; k < 4; k++)
-            acc[k] += partial[4 * b + k];
-    for (int k = 0; k < 4; k++)
-        red[k][threadIdx.x] = acc[k];
-    __syncthreads();
-    for (int s = kThreads / 2; s > 0; s >>= 1)
+            v[k] = partial[4 * tid + k];
+    const double s = block_sum4(v, red);
+    if (tid < 64)
     {
-        if (static_cast<int>(threadIdx.x) < s)
-            for (int k = 0; k < 4; k++)
-                red[k][threadIdx.x] += red[k][threadIdx.x + s];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0)
-    {
-        const double sp = red[0][0], spp = red[1][0], so = red[2][0], soo = red[3][0];
+        const double sp = __shfl(s, 0), spp = __shfl(s, 1), so = __shfl(s, 2), soo = __shfl(s, 3);
         double std_pos = 0.0, std_out = 0.0;
         if (count > 1)
         {
@@ -186,33 +230,30 @@ __global__ __launch_bounds__(kThreads) void cfg_scale_kernel(const double* parti
             std_pos = sqrt(fmax(0.0, (spp - sp * sp / n) / (n - 1)));
             std_out = sqrt(fmax(0.0, (soo - so * so / n) / (n - 1)));
         }
-        factor[0] = 1.0f;
-        factor[1] = 0.0f;
-        if (std_out > 0.0)
+        if (tid == 0)
         {
-            factor[0] = static_cast<float>(static_cast<double>(rescale) * std_pos / std_out +
-                                           static_cast<double>(1.0f - rescale));
-            factor[1] = 1.0f;
+            const bool apply = std_out > 0.0;
+            factor[0] = apply ? static_cast<float>(static_cast<double>(rescale) * std_pos / std_out +
+                                                   static_cast<double>(1.0f - rescale))
+                              : 1.0f;
+            factor[1] = apply ? 1.0f : 0.0f;
         }
     }
     __syncthreads();
     if (factor[1] == 0.0f)
         return;
     const float f = factor[0];
-    const long long stride = 4LL * gridDim.x * kThreads;
-    for (long long i = 4 * (static_cast<long long>(blockIdx.x) * kThreads + threadIdx.x); i < count; i += stride)
+    const long long stride = 4LL * gridDim.x * kSumThreads;
+    for (; i + 4 <= count; i += stride)
     {
-        if (i + 4 <= count)
-        {
-            f4 o = *reinterpret_cast<const f4*>(out + i);
-            for (int e = 0; e < 4; e++)
-                o[e] *= f;
-            *reinterpret_cast<f4*>(out + i) = o;
-            continue;
-        }
-        for (long long k = i; k < count; k++)
-            out[k] *= f;
+        for (int e = 0; e < 4; e++)
+            o[e] *= f;
+        *reinterpret_cast<f4*>(out + i) = o;
+        if (i + stride + 4 <= count)
+            o = *reinterpret_cast<const f4*>(out + i + stride);
     }
+    for (long long k = i; k < count; k++)
+        out[k] *= f;
 }
 
 // sampler.cpp:253-263: x0 = x - bt * pred, xT = x + at * pred,
@@ -374,13 +415,14 @@ try
     if (!workspace || static_cast<int64_t>(workspace_bytes) < sv2_cfg_workspace_size(count))
         return set_error(SV2_EINVAL, "sv2_apply_cfg: the rescale needs sv2_cfg_workspace_size bytes of workspace");
     double* partial = static_cast<double*>(workspace);
-    const int nb = static_cast<int>(std::min<long long>(blocks_for(count), kReduceBlocks));
-    hipLaunchKernelGGL(cfg_sums_kernel, dim3(nb), dim3(kThreads), 0, stream, positive, negative, out,
+    const long long blocks = ((count + 3) / 4 + kSumThreads - 1) / kSumThreads;
+    const int nb = static_cast<int>(std::min<long long>(blocks, kReduceBlocks));
+    hipLaunchKernelGGL(cfg_sums_kernel, dim3(nb), dim3(kSumThreads), 0, stream, positive, negative, out,
                        static_cast<long long>(count), scale, partial);
     if ((rc = launch_status("cfg_sums_kernel launch")) != SV2_OK)
         return rc;
-    const int ns = static_cast<int>(std::min<long long>(blocks_for_quads(count), kScaleBlocks));
-    hipLaunchKernelGGL(cfg_scale_kernel, dim3(ns), dim3(kThreads), 0, stream, partial, nb, out,
+    const int ns = static_cast<int>(std::min<long long>(blocks, kScaleBlocks));
+    hipLaunchKernelGGL(cfg_scale_kernel, dim3(ns), dim3(kSumThreads), 0, stream, partial, nb, out,
                        static_cast<long long>(count), rescale);
     return launch_status("cfg_scale_kernel launch");
 }

@@ -204,3 +204,21 @@ def test_ragged_counts_and_alignments(sampler, orc, count, shift):
     sampler.apply_cfg(p, n, 6.5, 0.7, output=o)
     within_ulps(host(o), orc.apply_cfg(pos, neg, 6.5, 0.7))
     assert bool((box[:, :shift] == 7.0).all()) and bool((box[:, shift + count:] == 7.0).all())
+
+
+# a block's 4096 elements, the 512 blocks of the rescale and the 1024 of the
+# sums: one short of each, each, and past it
+@pytest.mark.parametrize("count", [4095, 4096, 4097, 4096 * 512, 4096 * 512 + 3, 4096 * 1024 - 1, 4096 * 1024 + 5])
+def test_rescale_around_the_grid_sizes(sampler, orc, count):
+    """The rescale where its kernels' blocks fill up and take a second quad a
+    thread, in place on the positive prediction, twice with the same bits."""
+    print(f"[rescale] count={count}", flush=True)
+    pos, neg = pair((count,), count % 1000)
+    neg_d = dev(neg)
+    outs = []
+    for _ in range(2):
+        p = dev(pos)
+        sampler.apply_cfg(p, neg_d, 6.5, 0.7, output=p)
+        outs.append(host(p))
+    within_ulps(outs[0], orc.apply_cfg(pos, neg, 6.5, 0.7))
+    assert np.array_equal(outs[0], outs[1])
