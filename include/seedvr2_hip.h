@@ -528,6 +528,24 @@ void sv2_dit_destroy(sv2_dit* dit);
 #define SV2_EPI_SWIGLU 2
 int sv2_inner_product_f16(const void* x, const void* w, const void* w_value, void* y, int rows, int in, int out,
                           int epilogue, const float* bias, const float* gate, const void* residual, void* stream);
+/* How an fp16 product of these sizes runs; launches nothing.  `block` 0:
+ * sv2_inner_product_f16 (SV2_EUNSUPPORTED for sizes it refuses); 1: the
+ * block's and heads' own products (param 14 = 0), which a rule on the sizes
+ * sends to the same kernel or to hipBLASLt.  The kernel computes the first
+ * first_rows rows (a multiple of 256, or 0) in 256 x 256 tiles and the rest in
+ * `form`; where `kernel` is 0 the same plan runs if hipBLASLt has no kernel for
+ * a residual product.  `form` is -1 for sizes the kernel does not take. */
+#define SV2_FORM_256X256 0
+#define SV2_FORM_256X128 1
+#define SV2_FORM_128X128 2
+#define SV2_FORM_128X128_KSPLIT 3 /* K split between the two wave groups */
+#define SV2_FORM_128X256 4        /* SwiGLU: 128 rows x (128 gate + 128 value) */
+typedef struct sv2_product_plan {
+    int kernel;     /* 1: the MFMA kernel (operands 16-byte aligned), 0: hipBLASLt */
+    int first_rows;
+    int form;
+} sv2_product_plan;
+int sv2_inner_product_f16_plan(int rows, int in, int out, int epilogue, int block, sv2_product_plan* plan);
 
 /* ---- The same InnerProducts and fused passes for 1-64 rows (the text
  * branch's tokens: seedvr2_dit_block.cpp:1155-1156, :1180-1181, :1101,

@@ -32,6 +32,7 @@ namespace
 {
 
 std::mutex g_mutex;
+constexpr const char* kNoKernel = "gemm: hipBLASLt has no workspace-free kernel for an fp16 product of this shape";
 
 int current_device(int* rc)
 {
@@ -169,7 +170,7 @@ int make_plan(hipblasLtHandle_t h, int rows, int in, int out, const Gated* gated
             return SV2_OK;
         }
     destroy_plan(plan);
-    return set_error(SV2_EUNSUPPORTED, "gemm: hipBLASLt has no workspace-free kernel for an fp16 product of this shape");
+    return set_error(SV2_EUNSUPPORTED, kNoKernel);
 }
 
 int gemm_f16(hipStream_t stream, int rows, int in, int out, const void* x, const void* w, void* y,
@@ -187,17 +188,17 @@ int gemm_f16(hipStream_t stream, int rows, int in, int out, const void* x, const
         if (!h)
             return rc;
         static std::map<PlanKey, LtPlan> plans;
-        static std::set<PlanKey> unsupported; // gated shapes the library has no kernel for
+        static std::set<PlanKey> unsupported; // shapes the library has no kernel for
         const PlanKey key{device, rows, in, out, gated ? (gated->bias ? 2 : 1) : 0};
         if (unsupported.count(key))
-            return set_error(SV2_EUNSUPPORTED, "gemm: hipBLASLt has no gated kernel for this shape");
+            return set_error(SV2_EUNSUPPORTED, kNoKernel);
         auto it = plans.find(key);
         if (it == plans.end())
         {
             LtPlan fresh;
             if ((rc = make_plan(h, rows, in, out, gated, &fresh)) != SV2_OK)
             {
-                if (gated && rc == SV2_EUNSUPPORTED)
+                if (rc == SV2_EUNSUPPORTED)
                     unsupported.insert(key);
                 return rc;
             }
@@ -263,9 +264,11 @@ int gemm_rows_bias(hipStream_t stream, int dtype, int rows, int in, int out, con
                               static_cast<float*>(y));
     if (dtype != SV2_F16)
         return set_error(SV2_EINVAL, "gemm: compute dtype must be fp32 or fp16");
-    const int rc = gemm_mfma_preferred(rows, in, out, kGemmStore, x, w, nullptr, y, nullptr)
-                       ? gemm_mfma(stream, rows, in, out, x, w, nullptr, y, kGemmStore, false, nullptr, nullptr, nullptr)
-                       : gemm_f16(stream, rows, in, out, x, w, y);
+    const bool preferred = gemm_mfma_preferred(rows, in, out, kGemmStore, x, w, nullptr, y, nullptr);
+    int rc = preferred ? SV2_EUNSUPPORTED : gemm_f16(stream, rows, in, out, x, w, y);
+    // also the sizes the library has no kernel without a workspace for
+    if (preferred || (rc == SV2_EUNSUPPORTED && gemm_mfma_fits(rows, in, out, kGemmStore, x, w, nullptr, y, nullptr)))
+        rc = gemm_mfma(stream, rows, in, out, x, w, nullptr, y, kGemmStore, false, nullptr, nullptr, nullptr);
     return (rc != SV2_OK || !bias) ? rc : launch_bias_rows(y, bias, SV2_F16, rows, out, stream);
 }
 

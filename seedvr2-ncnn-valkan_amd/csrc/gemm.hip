@@ -82,7 +82,7 @@ constexpr int kEpiWave = 16 * 128; // bytes of one wave's epilogue staging: 16 r
 constexpr int kEpiBytes = 8 * kEpiWave;
 constexpr int kMaxLds = 160 * 1024;
 constexpr int kCus = 256;            // compute units of one MI355X
-constexpr int kPreferRows = 256;
+constexpr int kPreferRows = 256;    // fewer rows go to the library
 constexpr int kTouchAhead = 3;      // stages before a tile's end
 constexpr float kLog2e = 1.4426950408889634f;
 
@@ -885,25 +885,68 @@ bool operands_fit(int rows, int in, int out)
     return static_cast<long long>(rows) * in * 2 <= INT_MAX && static_cast<long long>(out) * in * 2 <= INT_MAX;
 }
 
-// Whether a residual product is faster here than the library's product with
-// the residual in its epilogue.  Its 2560 columns make a third of qkv's tiles,
-// so most sizes leave CUs idle in the only or the last round, where the
-// library's tiles (192 x 256, 256 x 64 and others) divide better.  Inside a
-// block, out 6912 -> 2560 and proj 2560 -> 2560, library against this kernel:
-//   1018 rows   out 46 us / 61, proj 22 / 22      2065   78 / 97, 38 / 38
-//   4273        out 123 / 139, proj 60 / 68       10849  284 / 301, 124 / 139
-// This kernel wins where one round of `kSplit` tiles fills the CUs and K is
-// short (proj at 1361 rows 29 us / 22; at K = 6912 both take 60), and from two
-// whole 256 x 256 rounds with the third no less than a quarter full (17329
-// rows: out 506 / 472, proj 227 / 224; but 19489 rows, 3.01 rounds: 509 / 536,
-// 209 / 247).
+// Which products of the fp16 blocks take this kernel and which the library,
+// from both measured at 256 to 21658 rows with weights out of cache, against
+// the two hipBLASLt builds a process may map (torch's and ROCm's).  Figures:
+// library time / kernel time, torch's build and ROCm's.  SwiGLU, where the
+// library takes three launches, is 1.03 to 1.66 and 0.97 to 1.54 times as fast
+// on the kernel and always takes it.
+//
+// The kernel's tiles are 256 x 256 down to 128 x 128; the library has those
+// and others between, so it divides a product of few tiles better wherever
+// these leave CUs idle, and about as well where both run whole rounds.
+
+// qkv 2560 -> 7680 and its like.
+bool store_pays(int rows, int in, int out)
+{
+    // few stages: launch and epilogue are most of it, and shorter here
+    // (256 -> 768 1.1 to 1.8, 512 -> 1536 1.05 to 1.7, torch's build)
+    if (in <= 512)
+        return true;
+    // two whole rounds of 256 x 256 tiles or more: 0.97 to 1.28, 0.97 to 1.23
+    if (tiles_of(kBig, rows, out) >= 2 * kCus)
+        return true;
+    const Plan p = make_plan(rows, in, out, kGemmStore, false);
+    const long long tiles = tiles_of(p.rest, rows - p.first_rows, out);
+    // one round and a rest in smaller tiles: a rest of 60 tiles costs a launch
+    // and a round all the same (0.94 to 1.00, 0.98 to 1.06), 120 and more pay
+    // (0.95 to 1.23, 0.99 to 1.22)
+    if (p.first_rows > 0)
+        return 5 * tiles >= 2 * kCus;
+    // one round: up to 180 tiles 0.84 to 1.07, 0.76 to 1.12 (0.95, 0.91 on
+    // average); from 210 on 0.94 to 1.21, 0.95 to 1.23 (1.07, 1.09)
+    if (tiles <= kCus)
+        return 4 * tiles >= 3 * kCus;
+    // up to two rounds of 256 x 256 tiles: 390 tiles 0.92 to 1.02, 0.91 to
+    // 1.15; 420 and more 0.96 to 1.03, 0.98 to 1.23 (0.98, 1.10).  More than
+    // one round of a smaller tile runs below the large one's rate (720 tiles
+    // of 256 x 128 0.94 to 1.01; 3072 -> 9216 in 504 of 128 x 128 0.83)
+    return p.rest == kBig && 5 * tiles >= 8 * kCus;
+}
+
+// The products with a residual: proj 2560 -> 2560 and out 6912 -> 2560.  Their
+// few columns make a third of qkv's tiles, and the residual, read before a
+// tile's sums can leave, costs it 2 to 4 us.
 bool residual_pays(int rows, int in, int out)
 {
-    const long long split = tiles_of(kSplit, rows, out);
-    if (in <= out && split <= kCus && 10 * split >= 7 * kCus)
-        return true;
-    const long long big = tiles_of(kBig, rows, out);
-    return big / kCus >= 2 && 4 * (big % kCus) >= kCus;
+    const Plan p = make_plan(rows, in, out, kGemmResidual, false);
+    // one launch of the K-split form that fills the CUs, K long enough to hide
+    // the epilogue and short enough that 0.33 us a stage do not add up: proj in
+    // 200 to 240 tiles 1.00 to 1.08, 0.96 to 1.09, in 160 to 180 0.91 to 1.01,
+    // 0.89 to 0.98; 4096 -> 4096 0.99 to 1.10; but 1024 -> 1024 0.8, 1536 ->
+    // 1536 0.90 to 1.11 and 6912 -> 2560 0.97 to 1.19 (torch's build; ROCm's
+    // takes twice as long there)
+    if (p.first_rows == 0 && p.rest == kSplit && in >= 2048 && in <= 4096)
+    {
+        const long long split = tiles_of(kSplit, rows, out);
+        return split <= kCus && 4 * split >= 3 * kCus;
+    }
+    // K long against the epilogue, from nearly three rounds of 256 x 256 tiles
+    // on: out 0.94 to 1.19, 0.95 to 1.12 (1.06, 1.03 on average).  From two
+    // rounds to there it is 0.89 to 1.13, 0.94 to 1.06, by the luck of the
+    // library's choice, and before 0.55 to 1.09 with torch's build; proj 0.87 to
+    // 1.29, 0.88 to 1.02 from two rounds on and 0.57 to 1.02 before.
+    return in >= 6144 && 20 * tiles_of(kBig, rows, out) >= 57 * kCus;
 }
 
 } // namespace
@@ -927,8 +970,14 @@ bool gemm_mfma_preferred(int rows, int in, int out, int epi, const void* x, cons
 {
     // fewer rows leave most CUs without a tile; there the library's smaller
     // tiles are as fast (96 rows, 6912 -> 2560: 22 us against 48)
-    return rows >= kPreferRows && gemm_mfma_fits(rows, in, out, epi, x, w, w2, y, residual) &&
-           (epi != kGemmResidual || residual_pays(rows, in, out));
+    if (rows < kPreferRows || !gemm_mfma_fits(rows, in, out, epi, x, w, w2, y, residual))
+        return false;
+    switch (epi)
+    {
+    case kGemmStore: return store_pays(rows, in, out);
+    case kGemmResidual: return residual_pays(rows, in, out);
+    default: return true;
+    }
 }
 
 int gemm_mfma(hipStream_t stream, int rows, int in, int out, const void* x, const void* w, const void* w2, void* y,
@@ -988,3 +1037,27 @@ catch (...)
     return sv2::caught_exception("sv2_inner_product_f16");
 }
 
+extern "C" int sv2_inner_product_f16_plan(int rows, int in, int out, int epilogue, int block, sv2_product_plan* plan)
+try
+{
+    static_assert(SV2_FORM_256X256 == sv2::kBig && SV2_FORM_256X128 == sv2::kTall && SV2_FORM_128X128 == sv2::kSmall &&
+                      SV2_FORM_128X128_KSPLIT == sv2::kSplit && SV2_FORM_128X256 == sv2::kWide,
+                  "form codes of the C ABI and the kernel agree");
+    if (!plan || rows <= 0 || in <= 0 || out <= 0 ||
+        (epilogue != SV2_EPI_STORE && epilogue != SV2_EPI_RESIDUAL && epilogue != SV2_EPI_SWIGLU))
+        return sv2::set_error(SV2_EINVAL, "sv2_inner_product_f16_plan: bad sizes, epilogue or null pointer");
+    *plan = sv2_product_plan{0, 0, -1};
+    // a null operand is an aligned one: the sizes alone decide
+    if (!sv2::gemm_mfma_fits(rows, in, out, epilogue, nullptr, nullptr, nullptr, nullptr, nullptr))
+        return block ? SV2_OK
+                     : sv2::set_error(SV2_EUNSUPPORTED, "sv2_inner_product_f16_plan: sizes the kernel does not take");
+    const sv2::Plan p = sv2::make_plan(rows, in, out, epilogue, !block);
+    plan->kernel = !block || sv2::gemm_mfma_preferred(rows, in, out, epilogue, nullptr, nullptr, nullptr, nullptr, nullptr);
+    plan->first_rows = p.first_rows;
+    plan->form = p.rest;
+    return SV2_OK;
+}
+catch (...)
+{
+    return sv2::caught_exception("sv2_inner_product_f16_plan");
+}

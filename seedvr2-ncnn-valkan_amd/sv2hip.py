@@ -77,6 +77,7 @@ EXPORTS = [
     "sv2_dit_forward",
     "sv2_dit_destroy",
     "sv2_inner_product_f16",
+    "sv2_inner_product_f16_plan",
     "sv2_inner_product_f16_few_workspace",
     "sv2_inner_product_f16_few",
     "sv2_inner_product_f32",
@@ -329,6 +330,8 @@ def load() -> ctypes.CDLL:
     lib.sv2_dit_destroy.restype = None
     lib.sv2_inner_product_f16.argtypes = [vp, vp, vp, vp, i, i, i, i, vp, vp, vp, vp]
     lib.sv2_inner_product_f16.restype = i
+    lib.sv2_inner_product_f16_plan.argtypes = [i, i, i, i, i, vp]
+    lib.sv2_inner_product_f16_plan.restype = i
     lib.sv2_inner_product_f16_few_workspace.argtypes = [i, i, i, i]
     lib.sv2_inner_product_f16_few_workspace.restype = ctypes.c_int64
     lib.sv2_inner_product_f16_few.argtypes = [vp, vp, vp, vp, i, i, i, i, vp, vp, vp, vp, ctypes.c_size_t, vp]
@@ -1057,6 +1060,18 @@ def inner_product_f16(x, w, y, epilogue=EPI_STORE, w_value=None, bias=None, gate
                                        _ptr(bias), _ptr(gate), _ptr(residual), _stream(stream)),
           "sv2_inner_product_f16")
     return y
+
+
+TILE_FORMS = ("256x256", "256x128", "128x128", "128x128-ksplit", "128x256")
+
+
+def inner_product_f16_plan(rows, k, n, epilogue=EPI_STORE, block=False):
+    """(kernel, first_rows, form) of an fp16 product (sv2_inner_product_f16_plan):
+    whether the MFMA kernel runs it, the rows in 256 x 256 tiles before the
+    rest, and the rest's tile form (None: sizes the kernel does not take)."""
+    plan = (ctypes.c_int * 3)()
+    check(load().sv2_inner_product_f16_plan(rows, k, n, epilogue, int(block), plan), "sv2_inner_product_f16_plan")
+    return bool(plan[0]), plan[1], TILE_FORMS[plan[2]] if plan[2] >= 0 else None
 
 
 def inner_product_f16_few(x, w, y, epilogue=EPI_STORE, w_value=None, bias=None, gate=None, residual=None,
