@@ -86,18 +86,23 @@ def test_store(hip, rows, k, n):
     assert mean < 2e-4
 
 
-@pytest.mark.parametrize("rows,k,n", [
-    (1, 64, 256),        # one stage, one row of a tile
-    (128, 128, 512),     # two stages, fewer than any ring holds
-    (129, 192, 256),     # three stages, one row in the second tile
-    (700, 2560, 2560),   # 128 x 128 tiles
-    (960, 2560, 7680),   # 256 x 128 tiles
-    (2049, 1280, 7680),  # 256 x 256 tiles in one round, one row in the last band
-    (6700, 640, 2560),   # 256 x 256 tiles over one round, the last one short
-    (7300, 320, 7680),   # whole rounds of 256 x 256 tiles and a rest in another form
+@pytest.mark.parametrize("rows,k,n,first,form", [
+    (1, 64, 256, 0, "128x128"),        # one stage, one row of a tile
+    (128, 128, 512, 0, "128x128"),     # two stages, fewer than any ring holds
+    (129, 192, 256, 0, "128x128"),     # three stages, one row in the second tile
+    (700, 2560, 2560, 0, "128x128"),
+    (2049, 1280, 7680, 0, "128x128"),  # four rounds, one row in the last band
+    (960, 2560, 7680, 0, "256x128"),
+    (6700, 640, 2560, 0, "256x128"),   # over two rounds, the last one short
+    (1793, 1280, 7680, 0, "256x256"),  # one round, one row in the last band
+    (7300, 320, 7680, 0, "256x256"),   # over three rounds, the last one short
+    (2305, 1280, 7680, 2048, "128x128"),  # a round of 256 x 256 tiles and a rest of one row past two bands
+    (7300, 1280, 7680, 6400, "256x128"),
 ])
-def test_store_tile_forms(hip, rows, k, n):
-    """The tile forms and the edges of their ranges; rows past the output stay untouched."""
+def test_store_tile_forms(hip, rows, k, n, first, form):
+    """The tile forms and the edges of their ranges, and rows in 256 x 256
+    tiles with the rest in another form; rows past the output stay untouched."""
+    assert hip.inner_product_f16_plan(rows, k, n) == (True, first, form)
     print(f"[tile form] rows={rows} in={k} out={n}", flush=True)
     gen = torch.Generator(device="cuda").manual_seed(rows * 3 + k + n)
     x = rand16((rows, k), 1.0, gen)
@@ -154,6 +159,29 @@ def test_swiglu(hip, rows, k, f):
     assert_ulp(y.float().cpu().numpy(), ref)
 
 
+@pytest.mark.parametrize("rows,k,f,first,form", [
+    (257, 64, 256, 0, "128x256"),       # one stage, one row in the last band
+    (1000, 2560, 6912, 0, "256x256"),
+    (1361, 2560, 6912, 1024, "128x256"),  # a round of 256 x 256 tiles and a ragged rest
+])
+def test_swiglu_tile_forms(hip, rows, k, f, first, form):
+    """SwiGLU in each of its forms; rows past the output stay untouched."""
+    assert hip.inner_product_f16_plan(rows, k, f, hip.EPI_SWIGLU) == (True, first, form)
+    gen = torch.Generator(device="cuda").manual_seed(rows + f)
+    x = rand16((rows, k), 1.0, gen)
+    wg, wu = rand16((f, k), 0.02, gen), rand16((f, k), 0.02, gen)
+    pg = torch.empty((rows, f), dtype=torch.float16, device="cuda")
+    pu = torch.empty_like(pg)
+    y = torch.full((rows + 2, f), 7.0, dtype=torch.float16, device="cuda")
+    hip.inner_product_f16(x, wg, pg)
+    hip.inner_product_f16(x, wu, pu)
+    hip.inner_product_f16(x, wg, y[:rows], hip.EPI_SWIGLU, w_value=wu)
+    torch.cuda.synchronize()
+    assert bool((y[rows:] == 7.0).all())
+    gg, uu = pg.float().cpu().numpy(), pu.float().cpu().numpy()
+    assert_ulp(y[:rows].float().cpu().numpy(), ((gg / (np.float32(1.0) + np.exp(-gg))) * uu).astype(np.float16))
+
+
 @pytest.mark.parametrize("rows", [64, 256])
 def test_swiglu_as_exact_as_expf_and_a_divide(hip, rows):
     """silu(g) u of the entry point (`rounded` products) to fp32 accuracy: with
@@ -196,12 +224,11 @@ def test_unsupported_shapes(hip):
 
 
 def test_x_operand_just_under_2gib(hip):
-    """X of (2^24 - 100) rows x 64 in: 2 GiB less 12.8 KB, the largest kind of
-    operand the 32-bit buffer offsets admit, with a ragged last row tile whose
-    padded rows' offsets pass INT_MAX (formed unsigned in the kernel, and
-    returned as zeros by the buffer resource).  Rows at the start, around the
-    2^30-byte and 2^31 - 1 marks and at the end against the float64
-    product."""
+    """X of (2^24 - 100) rows x 64 in: 2 GiB less 12.8 KB, about the largest
+    operand the entry point takes, with a ragged last row tile whose rows past
+    the end repeat the last one (a tile's base is a 64-bit address, its rows
+    32-bit offsets from it).  Rows at the start, around the 2^30-byte and
+    2^31 - 1 marks and at the end against the float64 product."""
     rows, k, n = (1 << 24) - 100, 64, 256
     print(f"[gemm] rows={rows} k={k} n={n} (X {rows * k * 2 / 2**30:.4f} GiB)", flush=True)
     gen = torch.Generator(device="cuda").manual_seed(5)
