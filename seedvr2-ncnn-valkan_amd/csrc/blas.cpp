@@ -2,12 +2,14 @@
 //
 // fp16 (the fast mode), fp32 accumulation: gemm_mfma (gemm.hip) where
 // gemm_mfma_preferred says so, by the sizes and alignments alone; else
-// hipBLASLt.  The first library product of a shape on a device plans it: the
-// library's best-ranked kernel that needs no workspace, kept for the rest of
-// the process.  The choice depends on the shape alone, so a shape is computed
-// with the same kernel (and rounds the same way) in every process, and
-// planning neither runs nor synchronises anything.  (Timing the library's 16 best-ranked kernels instead and keeping
-// the fastest changed the 720p DiT step by less than its run-to-run spread.)
+// hipBLASLt, and gemm_mfma again for sizes that one has no kernel for.  The
+// first library product of a shape on a device plans it: the library's
+// best-ranked kernel that needs no workspace, kept for the rest of the
+// process.  The choice depends on the shape alone, so a shape is computed with
+// the same kernel (and rounds the same way) in every process, and planning
+// neither runs nor synchronises anything.  (Timing the library's 16 best-ranked
+// kernels instead and keeping the fastest changed the 720p DiT step by less
+// than its run-to-run spread.)
 // Without a workspace, products on different streams share nothing.  The
 // gated form carries the block's gated residual in the library's epilogue
 // (per-channel alpha, beta 1, optional bias), planned per shape in the same

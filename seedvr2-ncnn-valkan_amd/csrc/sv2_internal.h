@@ -159,7 +159,8 @@ int launch_residual_table(void* x, const void* residual, int dtype, int rows, in
 // y[rows, out] = x[rows, in] W^T, W [out][in] row-major (an InnerProduct
 // without its bias), in dtype (SV2_F32 or SV2_F16); enqueued on `stream`.
 // fp16 runs with fp32 accumulation on gemm_mfma where gemm_mfma_preferred says
-// so, else on hipBLASLt; fp32 on gemm_f32_exact.
+// so or hipBLASLt has no kernel for the sizes, else on hipBLASLt; fp32 on
+// gemm_f32_exact.
 int gemm_rows(hipStream_t stream, int dtype, int rows, int in, int out, const void* x, const void* w, void* y);
 // The same with the InnerProduct's bias (may be NULL): fp32 adds it to the
 // double sum before the one rounding; fp16 adds it in a pass after the product.
@@ -172,7 +173,8 @@ int gemm_f32_exact(hipStream_t stream, int rows, int in, int out, const float* x
 // fp16 only: y = gate[c] * (x W^T)[r][c] + residual[r][c] (+ bias[c] when
 // bias is not null), the gated residual of seedvr2_dit_block.cpp:807-825 in
 // the product's epilogue (fp32, one rounding to fp16), on gemm_mfma or
-// hipBLASLt as gemm_rows; -2 when hipBLASLt has no kernel for it.  A preceding InnerProduct bias b enters as bias = gate * b.
+// hipBLASLt as gemm_rows; SV2_EUNSUPPORTED where neither takes the sizes.  A
+// preceding InnerProduct bias b enters as bias = gate * b.
 int gemm_rows_gated(hipStream_t stream, int dtype, int rows, int in, int out, const void* x, const void* w, void* y,
                     const float* gate, const void* residual, const float* bias = nullptr);
 

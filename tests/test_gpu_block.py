@@ -628,12 +628,14 @@ def test_fp16_products_around_the_kernel_choice(hip, orc, device, grid, L):
 
 
 def test_fp16_residual_products_on_split_tiles(hip, orc, device):
-    """5768 rows at width 512: the residual products take one round of 128 x 128
-    tiles with K split between the wave groups (184 tiles, a ragged last band);
-    against the oracle."""
-    T, H, W, L = 6, 31, 31, 2
-    dim, heads, hidden = 512, 4, 512
-    rng = np.random.default_rng(5768)
+    """1224 video rows at the model's width: proj with its residual in one launch of
+    128 x 128 tiles with K split between the wave groups (200 tiles, 72 rows in
+    the last band); against the oracle."""
+    T, H, W, L = 1, 34, 36, 27
+    dim, heads, hidden = 2560, 20, 512
+    assert hip.inner_product_f16_plan(T * H * W, dim, dim, hip.EPI_RESIDUAL, block=True) == (
+        True, 0, "128x128-ksplit")
+    rng = np.random.default_rng(1224)
     w = nf.random_weights(rng, dim, hidden, shared=True)
     rows = rng.standard_normal((T * H * W + L, dim), dtype=np.float32).astype(np.float16).astype(np.float32)
     emb = rng.standard_normal(6 * dim, dtype=np.float32)
@@ -643,3 +645,57 @@ def test_fp16_residual_products_on_split_tiles(hip, orc, device):
         compare(hip, orc, blk, w, rows[:T * H * W], rows[T * H * W:], emb, T, H, W, device, "split tiles")
     finally:
         blk.close()
+
+
+# (grid, text rows): merged row counts at which hipBLASLt (torch's build) has
+# no workspace-free kernel for one product or another - 7233, 11841, 14401,
+# 16481 and 16961 (qkv, gate, or out, whose refusal moves it to the MFMA
+# kernel) -, 10881, and 20161, where out takes 256 x 256 tiles and a K-split rest
+ROW_COUNTS = [((6, 30, 40), 33), ((5, 46, 47), 71), ((5, 48, 49), 81), ((6, 48, 50), 1), ((4, 64, 64), 97),
+              ((6, 47, 60), 41), ((6, 55, 61), 31)]
+
+
+@pytest.fixture(scope="module")
+def wide_blocks(hip):
+    """A shared-weights block at the model's sizes with the products by the
+    size rule, and one with all of them on the MFMA kernel, whose products are
+    rounded before each pass (held to the oracle above)."""
+    gen = torch.Generator(device="cuda").manual_seed(77)
+    dim, hidden = 2560, 6912
+    shapes = {"attn_shift": (dim,), "attn_scale": (dim,), "attn_gate": (dim,), "mlp_shift": (dim,), "mlp_scale": (dim,),
+              "mlp_gate": (dim,), "w_qkv": (3 * dim, dim), "w_proj": (dim, dim), "b_proj": (dim,),
+              "w_gate": (hidden, dim), "w_in": (hidden, dim), "w_out": (dim, hidden)}
+    vid = {k: (torch.randn(s, generator=gen, device="cuda") * 0.02).to(torch.float16 if len(s) == 2 else torch.float32)
+           for k, s in shapes.items()}
+    vid["norm_q"], vid["norm_k"] = (torch.rand(128, generator=gen, device="cuda") + 0.5 for _ in range(2))
+    w = {"vid": vid, "freqs": nf.random_weights(np.random.default_rng(0), 128, 128, shared=True)["freqs"]}
+    made = [hip.DitBlock.from_device(hip.block_config(shared_weights=1, shifted_window=0, block_index=10, fused_gemm=f),
+                                     w, hip.F16) for f in (0, 1)]
+    yield made
+    for blk in made:
+        blk.close()
+
+
+@pytest.mark.parametrize("grid,L", ROW_COUNTS, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_fp16_block_at_row_counts_the_library_refuses(hip, wide_blocks, grid, L):
+    """The forward runs and agrees with the one whose products are all on the
+    MFMA kernel: each within 1e-3 (NRMSE) of the exact block, so 2e-3 of each
+    other."""
+    n = grid[0] * grid[1] * grid[2]
+    routes = [hip.inner_product_f16_plan(n + L, k, c, e, block=True) for k, c, e in (
+        (2560, 7680, hip.EPI_STORE), (2560, 2560, hip.EPI_RESIDUAL), (2560, 6912, hip.EPI_SWIGLU),
+        (6912, 2560, hip.EPI_RESIDUAL))]
+    print(f"[refused rows] {n + L}: {routes}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(n + L)
+    x = torch.randn((n + L, 2560), generator=gen, device="cuda").half()
+    emb = torch.randn(6 * 2560, generator=gen, device="cuda")
+    outs = []
+    for blk in wide_blocks:
+        blk.set_runtime_shape(*grid)
+        out = torch.full_like(x, float("nan"))
+        blk.forward(x[:n], x[n:], emb, out[:n], out[n:])
+        torch.cuda.synchronize()
+        assert blk.last_forward_merged()
+        outs.append(out.float())
+    assert bool(torch.isfinite(outs[0]).all())
+    assert float((outs[0] - outs[1]).norm() / outs[1].norm()) <= TOL_NRMSE

@@ -62,3 +62,16 @@ def test_plan_argument_checks(hip):
     assert f(4, 48, 256, hip.EPI_STORE, 0, plan) == hip.SV2_EUNSUPPORTED
     assert f(1 << 24, 64, 256, hip.EPI_STORE, 0, plan) == hip.SV2_EUNSUPPORTED  # X of 2 GiB
     assert f(4, 48, 256, hip.EPI_STORE, 1, plan) == hip.SV2_OK and plan[0] == 0 and plan[2] == -1
+
+
+def test_forms_of_the_residual_products(hip):
+    """The forms the blocks' residual products reach: proj in one launch of
+    K-split tiles, out in 256 x 256 tiles alone, with a K-split rest and with a
+    256 x 128 one; and a count (16961) that is the library's, whose build in
+    torch has no kernel for out there."""
+    plan = lambda rows, k: hip.inner_product_f16_plan(rows, k, 2560, hip.EPI_RESIDUAL, block=True)
+    assert plan(1224, 2560) == (True, 0, "128x128-ksplit")
+    assert plan(18881, 6912) == (True, 0, "256x256")
+    assert plan(20161, 6912) == (True, 19456, "128x128-ksplit")
+    assert plan(21658, 6912) == (True, 19456, "256x128")
+    assert plan(16961, 6912) == (False, 0, "256x256")
