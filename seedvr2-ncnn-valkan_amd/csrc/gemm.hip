@@ -198,9 +198,6 @@ __device__ inline void wait_younger(int n)
 {
     switch (n)
     {
-    case 18: wait_vm<18>(); break;
-    case 16: wait_vm<16>(); break;
-    case 14: wait_vm<14>(); break;
     case 12: wait_vm<12>(); break;
     case 8: wait_vm<8>(); break;
     case 6: wait_vm<6>(); break;
@@ -657,9 +654,11 @@ __global__ __launch_bounds__(kThreads) void gemm_tile_kernel(TileArgs a)
         int m0, n0;
         tile_of(tile, &m0, &n0);
         int i = 0;
-        if constexpr (EPI == kGemmResidual)
+        if constexpr (EPI == kGemmResidual && MH == 2)
         {
-            // the tile's residual lines move into the L2 while its last stages run
+            // the tile's residual lines move into the L2 while its last stages
+            // run (not for the 128 x 128 forms, whose waves have half a
+            // touch's rows each)
 #pragma nounroll
             for (; i < steady - kTouchAhead; i++)
                 stage(std::true_type{}, g++);
@@ -788,8 +787,8 @@ double form_us(Form f, int rows, int in, long long wrows)
 // alone.
 struct Plan
 {
-    Form first, rest;
-    int first_rows; // 0: all rows in `rest`
+    int first_rows; // in 256 x 256 tiles; 0: all rows in `rest`
+    Form rest;
     double us;
 };
 
@@ -805,23 +804,20 @@ Plan make_plan(int rows, int in, int out, int epi, bool rounded)
     }
     else
     {
-        if (out % 256 == 0)
-            forms[nf++] = kBig;
+        forms[nf++] = kBig;
         forms[nf++] = kTall;
         forms[nf++] = kSmall;
         // the rounded epilogues keep one order of summation in every form
         if (!rounded)
             forms[nf++] = kSplit;
     }
-    Plan best{kBig, forms[0], 0, form_us(forms[0], rows, in, wrows)};
+    Plan best{0, kBig, form_us(kBig, rows, in, wrows)};
     for (int i = 1; i < nf; i++)
     {
         const double us = form_us(forms[i], rows, in, wrows);
         if (us < best.us)
-            best = Plan{kBig, forms[i], 0, us};
+            best = Plan{0, forms[i], us};
     }
-    if (forms[0] != kBig)
-        return best;
     const long long per_band = wrows / 256;
     const long long bands = static_cast<long long>(kCus) * (tiles_of(kBig, rows, wrows) / kCus) / per_band;
     const long long first = bands * 256;
@@ -831,7 +827,7 @@ Plan make_plan(int rows, int in, int out, int epi, bool rounded)
             const double us = form_us(kBig, static_cast<int>(first), in, wrows) +
                               form_us(forms[i], rows - static_cast<int>(first), in, wrows);
             if (us < best.us)
-                best = Plan{kBig, forms[i], static_cast<int>(first), us};
+                best = Plan{static_cast<int>(first), forms[i], us};
         }
     return best;
 }
@@ -1010,7 +1006,7 @@ int gemm_mfma(hipStream_t stream, int rows, int in, int out, const void* x, cons
     const Plan plan = make_plan(rows, in, out, epi, rounded);
     if (plan.first_rows > 0)
     {
-        const int rc = run_rows(plan.first, a, epi, 0, plan.first_rows, stream);
+        const int rc = run_rows(kBig, a, epi, 0, plan.first_rows, stream);
         if (rc != SV2_OK)
             return rc;
     }
