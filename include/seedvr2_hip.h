@@ -253,7 +253,9 @@ typedef struct sv2_block_config {
                             proj_out + gated residual; gate/in + SwiGLU; out + gated residual),
                             fp16 compute only (ignored for fp32) and not while debug captures
                             are set; needs dim % 256 == 0 and mlp_hidden % 128 == 0.
-                            0 (default) = library GEMMs and separate passes. */
+                            0 (default) = each fp16 product on that kernel or on hipBLASLt by
+                            its sizes (sv2_inner_product_f16_plan), rounded once after its
+                            fused pass. */
 } sv2_block_config;
 
 /* Weights of one branch ("vid", "txt" or the shared "all"), in the order the
@@ -519,7 +521,8 @@ void sv2_dit_destroy(sv2_dit* dit);
  *                     the gate of apply_mlp (:1093-1112)
  * x fp16 [rows, in]; W, W_value fp16 [out, in] row-major (the InnerProduct
  * weight layout); residual fp16 [rows, out]; bias, gate fp32 [out].  Every
- * fp32 step follows the unfused kernels' order.  Requires in % 64 == 0 and
+ * fp32 step follows the unfused passes' order; silu is expf and an IEEE
+ * divide (2.5 fp32 ulps).  Requires in % 64 == 0 and
  * out % 256 == 0 (SV2_EPI_SWIGLU: out % 128 == 0); SV2_EUNSUPPORTED
  * otherwise.  x, W, W_value, y and residual must be 16-byte aligned
  * (SV2_EINVAL otherwise).  y may not alias x, W or residual. */

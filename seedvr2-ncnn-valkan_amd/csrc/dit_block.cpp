@@ -2,9 +2,9 @@
 // of the reference): parameters, weight loading from the exported
 // .param/.bin pair, and the block forward as a chain of the library's kernels
 // on one stream — token RMSNorm + ada, the QKV / proj / MLP InnerProducts
-// (hipBLASLt in fp16, the fp64-accumulating exact GEMM in the fp32 parity
-// mode, or the fused MFMA kernel under param 14), the windowed attention,
-// gated residuals and SwiGLU.
+// (fp16: the fused MFMA kernel or hipBLASLt by their sizes, the former for all
+// of them under param 14; the fp64-accumulating exact GEMM in the fp32 parity
+// mode), the windowed attention, gated residuals and SwiGLU.
 #include <algorithm>
 #include <cstring>
 #include <string>

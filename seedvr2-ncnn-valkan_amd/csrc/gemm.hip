@@ -29,22 +29,26 @@
 // runs; the ring runs on across tiles, so a tile's first stages are in flight
 // during the epilogue of the one before.  Outputs leave with non-temporal
 // stores: written through the L2 they evict the operand panels (128 KB a tile
-// and CU is the whole L2 of an XCD), qkv at 21658 rows 758 us against 667.
+// and CU is the whole L2 of an XCD), and qkv at 21658 rows takes an eighth
+// longer.
 //
-// What bounds it, 21658 rows (MI355X; the library product beside it):
-//   qkv 2560 -> 7680                   594 us (1.43 PFLOP/s)   589
-//   proj 2560 -> 2560 + residual       250 us                  276
-//   gate/in 2560 -> 2 x 6912 + SwiGLU  1062 us                 1067 + 137
-//   out 6912 -> 2560 + residual        605 us                  676
-// With all-zero operands the same launches take 434 / 215 / 773 / 512 us: on
-// random data the clock drops under the matrix cores' power, and the rest is
-// LDS bandwidth (192 KB of operand reads and 64 KB of fetch a 256 x 256 stage,
-// 2048 cycles at 128 B/clk, as many as its MFMAs take).  A 128 x 128 tile
-// reads three bytes of LDS where the large one reads two, and runs at 0.39 us
-// a stage against 0.24 us for a quarter of the large one's; it is there for
-// the products that would leave CUs idle.  `KS` is the 128 x 128 tile with a
-// 64 x 64 part per wave: the two groups take one k-step of each stage each and
-// add their sums at the end (reads a third less LDS than 64 x 32 parts do).
+// What bounds it, 21658 rows in a block (MI355X, kernel trace, us; the library
+// beside it, its separate SwiGLU pass after the +):
+//   qkv 2560 -> 7680                   609 (1.40 PFLOP/s)   606
+//   proj 2560 -> 2560 + residual       282                  281
+//   gate/in 2560 -> 2 x 6912 + SwiGLU  1109                 1076 + 135
+//   out 6912 -> 2560 + residual        620                  629
+// The matrix cores are busy 71 to 77% of the cycles of a 256 x 256 launch, at
+// 1.7 GHz: with all-zero operands, alone and back to back, the four take 434 /
+// 215 / 773 / 512 us, with random ones 594 / 250 / 1062 / 605, where the clock
+// drops under the matrix cores' power.  The rest is LDS bandwidth (192 KB of
+// operand reads and 64 KB of fetch a 256 x 256 stage, 2048 cycles at 128
+// B/clk, as many as its MFMAs take).  A 128 x 128 tile reads three bytes of LDS
+// where the large one reads two, and runs at 0.39 us a stage against 0.24 us
+// for a quarter of the large one's; it is there for the products that would
+// leave CUs idle.  `KS` is the 128 x 128 tile with a 64 x 64 part per wave: the
+// two groups take one k-step of each stage each and add their sums at the end
+// (reads a third less LDS than 64 x 32 parts do).
 //
 // Epilogues, in fp32 from the accumulators:
 //   kGemmStore     Y = fp16(acc)

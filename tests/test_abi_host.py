@@ -203,8 +203,8 @@ def test_elementwise_argument_checks(hip):
 def test_inner_product_argument_checks(hip):
     """Shape, pointer and size checks of the InnerProduct entry points return
     before any launch: the hand-written fp16 product needs in % 64 == 0 and
-    out % 256 == 0 (SwiGLU: % 128), and refuses operands past 2 GiB (its
-    buffer resources take 32-bit byte offsets); the fp32 exact product needs
+    out % 256 == 0 (SwiGLU: % 128), and refuses operands past 2 GiB (its row
+    offsets take 32 bits); the fp32 exact product needs
     positive sizes."""
     lib = hip.load()
     p = 16  # a non-null dummy address: every case below returns before touching it

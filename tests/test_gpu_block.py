@@ -2,7 +2,7 @@
 restatement of the reference CPU forward (seedvr2_dit_block.cpp:1114-1267).
 
 The block chains token RMSNorm + ada, the QKV / proj / MLP InnerProducts
-(hipBLASLt in fp16; in the fp32 mode a GEMM accumulating in double in the
+(fp16: the MFMA kernel or hipBLASLt by size; fp32: a GEMM accumulating in double in the
 oracle's order), the windowed attention kernel (the exact kernel in the fp32
 mode), the gated residuals and SwiGLU.  Gates:
   * fp32 compute mode (the parity mode, which computes the reference CPU
