@@ -100,22 +100,26 @@ __device__ inline float guide(float p, float n, float scale)
     return n + scaled;
 }
 
+// Grid-stride: a launch holds at most 2^32 threads, counts are not bounded by it.
 __global__ __launch_bounds__(kThreads) void cfg_kernel(const float* pos, const float* neg, float* out,
                                                        long long count, float scale)
 {
-    const long long i = 4 * (static_cast<long long>(blockIdx.x) * kThreads + threadIdx.x);
-    if (i + 4 <= count)
+    const long long stride = 4LL * gridDim.x * kThreads;
+    for (long long i = 4 * (static_cast<long long>(blockIdx.x) * kThreads + threadIdx.x); i < count; i += stride)
     {
-        const f4 p = *reinterpret_cast<const f4*>(pos + i);
-        const f4 n = *reinterpret_cast<const f4*>(neg + i);
-        f4 o;
-        for (int e = 0; e < 4; e++)
-            o[e] = guide(p[e], n[e], scale);
-        *reinterpret_cast<f4*>(out + i) = o;
-        return;
+        if (i + 4 <= count)
+        {
+            const f4 p = *reinterpret_cast<const f4*>(pos + i);
+            const f4 n = *reinterpret_cast<const f4*>(neg + i);
+            f4 o;
+            for (int e = 0; e < 4; e++)
+                o[e] = guide(p[e], n[e], scale);
+            *reinterpret_cast<f4*>(out + i) = o;
+            continue;
+        }
+        for (long long k = i; k < count; k++)
+            out[k] = guide(pos[k], neg[k], scale);
     }
-    for (long long k = i; k < count; k++)
-        out[k] = guide(pos[k], neg[k], scale);
 }
 
 // Lane l of the wave gets the sum over its lanes of v[l % 4]: two halving
@@ -408,8 +412,9 @@ try
     hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
     if (rescale == 0.0f)
     {
-        hipLaunchKernelGGL(cfg_kernel, dim3(blocks_for_quads(count)), dim3(kThreads), 0, stream, positive, negative,
-                           out, static_cast<long long>(count), scale);
+        const int nb = static_cast<int>(std::min<long long>(((count + 3) / 4 + kThreads - 1) / kThreads, 1LL << 20));
+        hipLaunchKernelGGL(cfg_kernel, dim3(nb), dim3(kThreads), 0, stream, positive, negative, out,
+                           static_cast<long long>(count), scale);
         return launch_status("cfg_kernel launch");
     }
     if (!workspace || static_cast<int64_t>(workspace_bytes) < sv2_cfg_workspace_size(count))

@@ -222,3 +222,19 @@ def test_rescale_around_the_grid_sizes(sampler, orc, count):
         outs.append(host(p))
     within_ulps(outs[0], orc.apply_cfg(pos, neg, 6.5, 0.7))
     assert np.array_equal(outs[0], outs[1])
+
+
+def test_guidance_past_the_threads_of_a_launch(sampler):
+    """2^34 + 5 elements (69 GB, in place on both predictions): more quads than
+    a launch can have threads.  With infinities on both sides every element
+    becomes NaN, and the guard behind them stays."""
+    count = (1 << 34) + 5
+    print(f"[guidance] count={count}", flush=True)
+    box = torch.full((count + 3,), float("inf"), device="cuda")
+    x = box[:count]
+    sampler.apply_cfg(x, x, 6.5, 0.0, output=x)
+    torch.cuda.synchronize()
+    assert all(bool(torch.isnan(x[i:i + (1 << 32)]).all()) for i in range(0, count, 1 << 32))
+    assert bool(torch.isinf(box[count:]).all())
+    del box, x
+    torch.cuda.empty_cache()
