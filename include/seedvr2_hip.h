@@ -537,7 +537,8 @@ int sv2_inner_product_f16(const void* x, const void* w, const void* w_value, voi
  * sends to the same kernel or to hipBLASLt.  The kernel computes the first
  * first_rows rows (a multiple of 256, or 0) in 256 x 256 tiles and the rest in
  * `form`; where `kernel` is 0 the same plan runs if hipBLASLt has no kernel for
- * a residual product.  `form` is -1 for sizes the kernel does not take. */
+ * the product (SwiGLU aside, which is then two products and a pass).  `form` is
+ * -1 for sizes the kernel does not take. */
 #define SV2_FORM_256X256 0
 #define SV2_FORM_256X128 1
 #define SV2_FORM_128X128 2
